@@ -70,7 +70,6 @@ constexpr int NPARAM = OFF_B5 + 4;  // 199,684
 constexpr int BF_SW = 0, BF_ROW = 3 * H * H, BF_SWLO = 6 * H * H, BF_TSW = 9 * H * H,
               BF_TSWLO = 12 * H * H;
 constexpr int NBF = 15 * H * H;
-constexpr int CP = 32;  // points per workgroup of tile_conservative
 
 // logistic function from the hardware exp2 and reciprocal (v_exp_f32,
 // v_rcp_f32, ~1 ulp each): the activations are rounded to BF16 (8 bits)
@@ -256,10 +255,10 @@ __device__ __forceinline__ void tile_forward(const float *__restrict__ theta, co
 constexpr int LDS_BYTES = TILE * LDSR * 2;
 
 // ---------------------------------------------------------------------------
-// The precise evaluation of one CP-point tile: o0 and d o0 / d f (reverse
-// mode), the hidden products in three BF16 matrix-core products of the
-// hi/lo split (hi*hi + hi*lo + lo*hi), SiLU and its derivative in FP32, the
-// first and last layers in FP32 on the VALU.
+// The precise evaluation of one tile of CP = 16 MI points: o0 and d o0 / d f
+// (reverse mode), the hidden products in three BF16 matrix-core products of
+// the hi/lo split (hi*hi + hi*lo + lo*hi), SiLU and its derivative in FP32,
+// the first and last layers in FP32 on the VALU.
 //   feat   LDS [CP][4] features;
 //   bhi,   LDS [CP][LDSR] BF16 each: a layer's input (activations forward,
 //   blo    error signals backward), split;
@@ -269,6 +268,20 @@ constexpr int LDS_BYTES = TILE * LDSR * 2;
 // Wave w owns units [64w, 64w + 64) of every layer (forward and backward),
 // so the SiLU derivatives it keeps in registers from the forward pass are
 // exactly those its reverse-pass products need.  All 256 threads call it.
+//
+// What bounds it: the matrix products and the SiLU arithmetic (1,152 MFMAs,
+// 18.4k cycles, and ~3,000 other vector instructions, ~15k cycles, per wave
+// and 32-point tile), with the weights' L2 reads (1.5 MB per tile) close
+// behind.  1,048,576 points take 2.41 ms, 1,040 TFLOP/s of executed BF16
+// products (a large library BF16 product reaches 1,150 on the same card); 3.91
+// ms while the layers were runtime loops, whose per-element branches kept the
+// derivatives in scratch memory and the weight reads inside each step.  Hence
+// every layer is written out (the derivatives stay in registers), and each
+// step's weights are read one step ahead, across the layers' barriers too.
+// Larger tiles halve the weight reads but leave one wave per SIMD (64 points:
+// 2.39 ms) or spill (48 points); 16-point tiles repeat them (3.58 ms) and only
+// pay while there are fewer tiles than compute units (4,096 points: 21 against
+// 24 us), see tile_points16.
 
 __device__ __forceinline__ void split_bf(float v, __bf16 &hi, __bf16 &lo) {
     hi = tobf(v);
@@ -277,147 +290,277 @@ __device__ __forceinline__ void split_bf(float v, __bf16 &hi, __bf16 &lo) {
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-// acc[mi][ni] (+)= sum over the 256 inputs of the layer's weights (fragment
-// order: hi at Whi, lo at Wlo) times the split input in bhi/blo
-__device__ __forceinline__ void split_layer(const __bf16 *__restrict__ Whi,
-                                            const __bf16 *__restrict__ Wlo, const __bf16 *bhi,
-                                            const __bf16 *blo, f32x4 (&acc)[2][4]) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// this thread's wave in its workgroup, as a scalar: addresses formed from it
+// stay in scalar registers
+__device__ __forceinline__ unsigned wave_id() {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+
+// The weights and parameters of the tile are read through buffer descriptors:
+// a 32-bit lane offset and a scalar offset per read, no 64-bit address
+// arithmetic on the vector unit.
+struct NetBufs {
+    __amdgpu_buffer_rsrc_t w, th;  // BF16 copies; FP32 parameters
+};
+__device__ __forceinline__ NetBufs net_bufs(const float *theta, const __bf16 *wbf) {
+    constexpr int FLAGS = 0x00027000;  // raw buffer, bounds-checked (gfx9 layout)
+    return {__builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16 *>(wbf), 0, NBF * 2, FLAGS),
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(theta), 0, NPARAM * 4, FLAGS)};
+}
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+// four consecutive parameters from index at (scalar) + lane_at
+__device__ __forceinline__ f32x4 theta4(const NetBufs &nb, unsigned at, unsigned lane_at) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(nb.th, lane_at * 4, at * 4, 0);
+    return __builtin_bit_cast(f32x4, v);
+}
+
+// one K step (32 inputs) of a wave's weight fragments from the layer blocks
+// at element offsets hi and lo: hi parts of its four 16-unit tiles in [0, 4),
+// lo parts in [4, 8)
+__device__ __forceinline__ void load_frags(bf16x8 (&f)[8], const NetBufs &nb, unsigned hi,
+                                           unsigned lo, int ks) {
+    const unsigned lane = threadIdx.x & 63, w = wave_id();
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-        for (int ni = 0; ni < 4; ni++) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int ks = 0; ks < 8; ks++) {
-        bf16x8 wh[4], wl[4];
-#pragma unroll
-        for (int ni = 0; ni < 4; ni++) {
-            const size_t o = (((size_t)(4 * w + ni) * 8 + ks) * 64 + lane) * 8;
-            wh[ni] = *reinterpret_cast<const bf16x8 *>(Whi + o);
-            wl[ni] = *reinterpret_cast<const bf16x8 *>(Wlo + o);
-        }
-#pragma unroll
-        for (int mi = 0; mi < 2; mi++) {
-            const int off = (16 * mi + (lane & 15)) * LDSR + 32 * ks + 8 * (lane >> 4);
-            const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(bhi + off);
-            const bf16x8 al = *reinterpret_cast<const bf16x8 *>(blo + off);
-#pragma unroll
-            for (int ni = 0; ni < 4; ni++) {
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[ni], ah, acc[mi][ni], 0, 0, 0);
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[ni], al, acc[mi][ni], 0, 0, 0);
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl[ni], ah, acc[mi][ni], 0, 0, 0);
-            }
-        }
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned o = ((4 * w + ni) * 8 + ks) * 64 * 8;
+        f[ni] = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(nb.w, lane * 16, (hi + o) * 2, 0));
+        f[4 + ni] = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(nb.w, lane * 16, (lo + o) * 2, 0));
     }
 }
 
+// acc[mi][ni] = sum over the 256 inputs of the layer's weights (fragment
+// order: hi parts at element whi of the copies, lo at wlo) times the split
+// input in bhi/blo.  The weights of step ks + 1 are loaded before step ks's
+// products; those of the first step are in f[0] on entry, and the next
+// layer's (nhi, nlo) are in f[0] on return, so that their latency passes
+// behind this layer's epilogue.
+template <int MI, bool NEXT>
+__device__ __forceinline__ void split_layer(const NetBufs &nb, unsigned whi, unsigned wlo,
+                                            unsigned nhi, unsigned nlo, const __bf16 *bhi,
+                                            const __bf16 *blo, bf16x8 (&f)[2][8],
+                                            f32x4 (&acc)[MI][4]) {
+    const unsigned lane = threadIdx.x & 63;
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < 4; ni++) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the matrix phase ahead of a neighbouring workgroup's SiLU phase (1 % of an
+    // orbit step)
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < 8; ks++) {
+        if (ks < 7)
+            load_frags(f[(ks + 1) & 1], nb, whi, wlo, ks + 1);
+        else if (NEXT)
+            load_frags(f[0], nb, nhi, nlo, 0);
+        __builtin_amdgcn_sched_barrier(0);  // one step of loads in flight, not all eight
+        const bf16x8(&w)[8] = f[ks & 1];
+        bf16x8 ah[MI], al[MI];
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++) {
+            const unsigned off = (16 * mi + (lane & 15)) * LDSR + 32 * ks + 8 * (lane >> 4);
+            ah[mi] = *reinterpret_cast<const bf16x8 *>(bhi + off);
+            al[mi] = *reinterpret_cast<const bf16x8 *>(blo + off);
+        }
+        // each accumulator takes hi*hi, hi*lo, lo*hi in that order; the three
+        // are issued 4 MI products apart, so none waits for the one before it
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int ni = 0; ni < 4; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[ni], ah[mi], acc[mi][ni], 0, 0, 0);
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int ni = 0; ni < 4; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[ni], al[mi], acc[mi][ni], 0, 0, 0);
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int ni = 0; ni < 4; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[4 + ni], ah[mi], acc[mi][ni], 0, 0, 0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+}
+
+// four consecutive units of one point, split, into the layer buffers
+__device__ __forceinline__ void store_split(__bf16 *bhi, __bf16 *blo, unsigned at, const float (&v)[4]) {
+    __bf16 hh[4], hl[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) split_bf(v[e], hh[e], hl[e]);
+    *reinterpret_cast<bf16x4 *>(bhi + at) = bf16x4{hh[0], hh[1], hh[2], hh[3]};
+    *reinterpret_cast<bf16x4 *>(blo + at) = bf16x4{hl[0], hl[1], hl[2], hl[3]};
+}
+
+// epilogue of hidden layer L (2..4): SiLU of acc + bias.  Layers 2 and 3 keep
+// their derivatives in ds and write the activations; layer 4 adds the
+// output dot to po and writes the output's error signal.
+template <int MI, int L>
+__device__ __forceinline__ void forward_epilogue(const NetBufs &nb,
+                                                 const f32x4 (&acc)[MI][4], __bf16 *bhi,
+                                                 __bf16 *blo, f32x4 (&ds)[MI][4],
+                                                 float (&po)[MI]) {
+    const unsigned lane = threadIdx.x & 63, w = wave_id();
+    constexpr unsigned bias = L == 2 ? OFF_B2 : L == 3 ? OFF_B3 : OFF_B4;
+    const unsigned lu = 4 * (lane >> 4);  // this lane's first unit of a 16-unit tile
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < 4; ni++) {
+            const unsigned unit = 64 * w + 16 * ni + 4 * (lane >> 4);
+            const unsigned row = 16 * mi + (lane & 15);
+            const f32x4 bc = theta4(nb, bias + 64 * w + 16 * ni, lu);
+            float out[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float z = acc[mi][ni][e] + bc[e];
+                const float sg = sigmoid_fast(z);
+                const float h = z * sg;
+                const float d = sg * (1.0f + z * (1.0f - sg));
+                if (L < 4) {
+                    ds[mi][ni][e] = d;
+                    out[e] = h;
+                } else {
+                    const float w5 = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   nb.th, lu * 16, (OFF_W5 + (64 * w + 16 * ni + e) * 4) * 4, 0));
+                    po[mi] += w5 * h;
+                    out[e] = w5 * d;
+                }
+            }
+            store_split(bhi, blo, row * LDSR + unit, out);
+        }
+}
+
+// epilogue of the reverse product into layer L - 1 = 3 or 2: the error signal
+template <int MI>
+__device__ __forceinline__ void reverse_epilogue(const f32x4 (&acc)[MI][4],
+                                                 const f32x4 (&ds)[MI][4], __bf16 *bhi,
+                                                 __bf16 *blo) {
+    const unsigned lane = threadIdx.x & 63, w = wave_id();
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < 4; ni++) {
+            const unsigned unit = 64 * w + 16 * ni + 4 * (lane >> 4);
+            const unsigned row = 16 * mi + (lane & 15);
+            float out[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) out[e] = acc[mi][ni][e] * ds[mi][ni][e];
+            store_split(bhi, blo, row * LDSR + unit, out);
+        }
+}
+
+template <int MI>
 __device__ __forceinline__ void tile_conservative(const float *__restrict__ theta,
                                                   const __bf16 *__restrict__ wbf,
                                                   const float (*feat)[4], __bf16 *bhi, __bf16 *blo,
-                                                  float (*red)[CP][5], float *o0, float (*dfo)[4]) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    // layer 1 (FP32): thread t owns unit t
+                                                  float (*red)[16 * MI][5], float *o0,
+                                                  float (*dfo)[4]) {
+    constexpr int NP = 16 * MI;  // points of the tile
+    const unsigned t = threadIdx.x, lane = t & 63, w = wave_id();
+    constexpr unsigned Fhi = BF_SW, Flo = BF_SWLO;    // forward, layers 2..4
+    constexpr unsigned Rhi = BF_TSW, Rlo = BF_TSWLO;  // their transposes
+    constexpr unsigned LW = H * H;
+    const NetBufs nb = net_bufs(theta, wbf);
+    bf16x8 f[2][8];
+    load_frags(f[0], nb, Fhi, Flo, 0);
+    // layer 1 (FP32): thread t owns units 2j and 2j + 1, j = t % 128, of half
+    // of the points
     {
-        const int j = t;
-        const float w0 = theta[OFF_W1 + 0 * H + j], w1 = theta[OFF_W1 + 1 * H + j];
-        const float w2 = theta[OFF_W1 + 2 * H + j], w3 = theta[OFF_W1 + 3 * H + j];
-        const float bj = theta[OFF_B1 + j];
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const unsigned j = 2 * (t & 127);
+        const f32x2 w0 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 0 * H + j);
+        const f32x2 w1 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 1 * H + j);
+        const f32x2 w2 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 2 * H + j);
+        const f32x2 w3 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 3 * H + j);
+        const f32x2 bj = *reinterpret_cast<const f32x2 *>(theta + OFF_B1 + j);
+        const unsigned p0 = (t >> 7) * (NP / 2);
 #pragma unroll 4
-        for (int p = 0; p < CP; p++) {
-            const float z = bj + feat[p][0] * w0 + feat[p][1] * w1 + feat[p][2] * w2 + feat[p][3] * w3;
-            split_bf(silu(z), bhi[p * LDSR + j], blo[p * LDSR + j]);
+        for (unsigned p = p0; p < p0 + NP / 2; p++) {
+            const f32x4 fp = *reinterpret_cast<const f32x4 *>(feat[p]);
+            __bf16 hh[2], hl[2];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const float z = bj[e] + fp[0] * w0[e] + fp[1] * w1[e] + fp[2] * w2[e] + fp[3] * w3[e];
+                split_bf(silu(z), hh[e], hl[e]);
+            }
+            *reinterpret_cast<bf16x2 *>(bhi + p * LDSR + j) = bf16x2{hh[0], hh[1]};
+            *reinterpret_cast<bf16x2 *>(blo + p * LDSR + j) = bf16x2{hl[0], hl[1]};
         }
     }
     __syncthreads();
     // SiLU derivatives of layers 2 and 3 at this wave's units, in the
     // accumulator layout: unit 64w + 16ni + 4(lane/16) + e, point 16mi + lane%16
-    f32x4 ds[2][2][4];
-    float po[2] = {0.f, 0.f};  // partial o0 of points lane%16 and 16 + lane%16
-    f32x4 acc[2][4];
-#pragma unroll 1
-    for (int l = 0; l < 3; l++) {
-        split_layer(wbf + BF_SW + (size_t)l * H * H, wbf + BF_SWLO + (size_t)l * H * H, bhi, blo,
-                    acc);
-        __syncthreads();  // every wave has read the layer's input
-        const float *bias = theta + (l == 0 ? OFF_B2 : l == 1 ? OFF_B3 : OFF_B4);
+    f32x4 ds2[MI][4], ds3[MI][4];
+    float po[MI];  // partial o0 of points 16mi + lane%16
+    f32x4 acc[MI][4];
 #pragma unroll
-        for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-            for (int ni = 0; ni < 4; ni++) {
-                const int unit = 64 * w + 16 * ni + 4 * (lane >> 4);
-                const int row = 16 * mi + (lane & 15);
-                const f32x4 bc = *reinterpret_cast<const f32x4 *>(bias + unit);
-                __bf16 hh[4], hl[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float z = acc[mi][ni][e] + bc[e];
-                    const float sg = sigmoid_fast(z);
-                    const float h = z * sg;
-                    const float d = sg * (1.0f + z * (1.0f - sg));
-                    if (l < 2) {
-                        ds[l][mi][ni][e] = d;
-                        split_bf(h, hh[e], hl[e]);
-                    } else {
-                        // layer 4: the output dot and the output's error signal
-                        const float w5 = theta[OFF_W5 + (unit + e) * 4];
-                        po[mi] += w5 * h;
-                        split_bf(w5 * d, hh[e], hl[e]);
-                    }
-                }
-                *reinterpret_cast<bf16x4 *>(bhi + row * LDSR + unit) = bf16x4{hh[0], hh[1], hh[2], hh[3]};
-                *reinterpret_cast<bf16x4 *>(blo + row * LDSR + unit) = bf16x4{hl[0], hl[1], hl[2], hl[3]};
-            }
-        __syncthreads();
-    }
+    for (int mi = 0; mi < MI; mi++) po[mi] = 0.f;
+    // every layer: the products, a barrier (every wave has read the layer's
+    // input), the epilogue into the same buffers, a barrier
+    split_layer<MI, true>(nb, Fhi, Flo, Fhi + LW, Flo + LW, bhi, blo, f, acc);
+    __syncthreads();
+    forward_epilogue<MI, 2>(nb, acc, bhi, blo, ds2, po);
+    __syncthreads();
+    split_layer<MI, true>(nb, Fhi + LW, Flo + LW, Fhi + 2 * LW, Flo + 2 * LW, bhi, blo, f, acc);
+    __syncthreads();
+    forward_epilogue<MI, 3>(nb, acc, bhi, blo, ds3, po);
+    __syncthreads();
+    split_layer<MI, true>(nb, Fhi + 2 * LW, Flo + 2 * LW, Rhi + 2 * LW, Rlo + 2 * LW, bhi, blo, f, acc);
+    __syncthreads();
+    forward_epilogue<MI, 4>(nb, acc, bhi, blo, ds3, po);
+    __syncthreads();
     // o0: the four lanes of a point in this wave, then the four waves
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++) {
+    for (int mi = 0; mi < MI; mi++) {
         float v = po[mi];
         v += __shfl_xor(v, 16);
         v += __shfl_xor(v, 32);
         if (lane < 16) red[w][16 * mi + lane][4] = v;
     }
     // reverse pass: delta_{l-1} = (W_l^T delta_l) silu'(z_{l-1}), l = 4, 3, 2
-    float pg[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 1
-    for (int l = 2; l >= 0; l--) {
-        split_layer(wbf + BF_TSW + (size_t)l * H * H, wbf + BF_TSWLO + (size_t)l * H * H, bhi, blo,
-                    acc);
-        __syncthreads();
+    split_layer<MI, true>(nb, Rhi + 2 * LW, Rlo + 2 * LW, Rhi + LW, Rlo + LW, bhi, blo, f, acc);
+    __syncthreads();
+    reverse_epilogue<MI>(acc, ds3, bhi, blo);
+    __syncthreads();
+    split_layer<MI, true>(nb, Rhi + LW, Rlo + LW, Rhi, Rlo, bhi, blo, f, acc);
+    __syncthreads();
+    reverse_epilogue<MI>(acc, ds2, bhi, blo);
+    __syncthreads();
+    split_layer<MI, false>(nb, Rhi, Rlo, 0, 0, bhi, blo, f, acc);
+    // layer 1's derivative, recomputed from its inputs, and d o0 / d f
+    float pg[MI][4];
+    f32x4 fr[MI];
 #pragma unroll
-        for (int mi = 0; mi < 2; mi++)
+    for (int mi = 0; mi < MI; mi++) {
+        fr[mi] = *reinterpret_cast<const f32x4 *>(feat[16 * mi + (lane & 15)]);
 #pragma unroll
-            for (int ni = 0; ni < 4; ni++) {
-                const int unit = 64 * w + 16 * ni + 4 * (lane >> 4);
-                const int row = 16 * mi + (lane & 15);
-                __bf16 hh[4], hl[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float d;
-                    if (l > 0) {
-                        d = acc[mi][ni][e] * ds[l - 1][mi][ni][e];
-                        split_bf(d, hh[e], hl[e]);
-                    } else {
-                        // layer 1's derivative, recomputed from its inputs
-                        const int u = unit + e;
-                        const float z = theta[OFF_B1 + u] + feat[row][0] * theta[OFF_W1 + u] +
-                                        feat[row][1] * theta[OFF_W1 + H + u] +
-                                        feat[row][2] * theta[OFF_W1 + 2 * H + u] +
-                                        feat[row][3] * theta[OFF_W1 + 3 * H + u];
-                        d = acc[mi][ni][e] * dsilu(z);
-#pragma unroll
-                        for (int c = 0; c < 4; c++) pg[mi][c] += theta[OFF_W1 + c * H + u] * d;
-                    }
-                }
-                if (l > 0) {
-                    *reinterpret_cast<bf16x4 *>(bhi + row * LDSR + unit) = bf16x4{hh[0], hh[1], hh[2], hh[3]};
-                    *reinterpret_cast<bf16x4 *>(blo + row * LDSR + unit) = bf16x4{hl[0], hl[1], hl[2], hl[3]};
-                }
-            }
-        __syncthreads();
+        for (int c = 0; c < 4; c++) pg[mi][c] = 0.f;
     }
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++)
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned tile = 64 * w + 16 * ni, lu = 4 * (lane >> 4);
+        f32x4 w1[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) w1[c] = theta4(nb, OFF_W1 + c * H + tile, lu);
+        const f32x4 b1 = theta4(nb, OFF_B1 + tile, lu);
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float z = b1[e] + fr[mi][0] * w1[0][e] + fr[mi][1] * w1[1][e] +
+                                fr[mi][2] * w1[2][e] + fr[mi][3] * w1[3][e];
+                const float d = acc[mi][ni][e] * dsilu(z);
+#pragma unroll
+                for (int c = 0; c < 4; c++) pg[mi][c] += w1[c][e] * d;
+            }
+    }
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             float v = pg[mi][c];
@@ -426,7 +569,7 @@ __device__ __forceinline__ void tile_conservative(const float *__restrict__ thet
             if (lane < 16) red[w][16 * mi + lane][c] = v;
         }
     __syncthreads();
-    if (t < CP) {
+    if (t < NP) {
         o0[t] = theta[OFF_B5] + red[0][t][4] + red[1][t][4] + red[2][t][4] + red[3][t][4];
 #pragma unroll
         for (int c = 0; c < 4; c++) dfo[t][c] = red[0][t][c] + red[1][t][c] + red[2][t][c] + red[3][t][c];
@@ -435,17 +578,19 @@ __device__ __forceinline__ void tile_conservative(const float *__restrict__ thet
 }
 
 // ---------------------------------------------------------------------------
-// inference: q (3,M) FP64 -> Phi_net (M), grad Phi_net (3,M), one CP-point
-// tile per workgroup (tile_conservative)
-__global__ __launch_bounds__(256) void k_mlp_forward(const float *__restrict__ theta,
+// inference: q (3,M) FP64 -> Phi_net (M), grad Phi_net (3,M), one tile of
+// 16 MI points per workgroup (tile_conservative)
+template <int MI>
+__global__ __launch_bounds__(256, 2) void k_mlp_forward(const float *__restrict__ theta,
                                                      const __bf16 *__restrict__ wbf,
                                                      gamd_mlp_norm nm,
                                                      const double *__restrict__ q, int64_t M,
                                                      double *__restrict__ phi,
                                                      double *__restrict__ grad) {
+    constexpr int CP = 16 * MI;  // points of the workgroup's tile
     __shared__ __align__(16) __bf16 bhi[CP * LDSR];
     __shared__ __align__(16) __bf16 blo[CP * LDSR];
-    __shared__ float feat[CP][4];
+    __shared__ __align__(16) float feat[CP][4];
     __shared__ float red[4][CP][5];
     __shared__ float o0[CP];
     __shared__ float dfo[CP][4];
@@ -464,7 +609,7 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const float *__restrict__ t
         for (int c = 0; c < 4; c++) feat[t][c] = f[c];
     }
     __syncthreads();
-    tile_conservative(theta, wbf, feat, bhi, blo, red, o0, dfo);
+    tile_conservative<MI>(theta, wbf, feat, bhi, blo, red, o0, dfo);
     if (t < CP && i < M) {
         double ph, gx, gy, gz;
         net_physics(nm, x, y, z, r, o0[t], dfo[t], ph, gx, gy, gz);
@@ -872,14 +1017,16 @@ __global__ void k_make_targets(gamd_mlp_norm nm, const double *__restrict__ q,
 // monitored energy Phi_net + |v|^2/2 is that of a conservative system; once
 // |E - E0| > tol |E0| the orbit switches to the exact SCF force for the rest
 // of the run (and for the remainder of this step).
-__global__ __launch_bounds__(256) void k_surrogate_step(
+template <int MI>
+__global__ __launch_bounds__(256, 2) void k_surrogate_step(
     const float *__restrict__ theta, const __bf16 *__restrict__ wbf, gamd_mlp_norm nm,
     double *__restrict__ wq, double *__restrict__ vsync, double *__restrict__ E0,
     int32_t *__restrict__ fb, double *__restrict__ wsw, int64_t N, double dt, int mode,
     int32_t step, double tol) {
+    constexpr int CP = 16 * MI;  // points of the workgroup's tile
     __shared__ __align__(16) __bf16 bhi[CP * LDSR];
     __shared__ __align__(16) __bf16 blo[CP * LDSR];
-    __shared__ float feat[CP][4];
+    __shared__ __align__(16) float feat[CP][4];
     __shared__ float red[4][CP][5];
     __shared__ float o0[CP];
     __shared__ float dfo[CP][4];
@@ -911,7 +1058,7 @@ __global__ __launch_bounds__(256) void k_surrogate_step(
     // the tile runs the network unless every orbit in it has fallen back
     // (uniform over the workgroup, so every thread reaches the same barriers)
     const int any_net = __syncthreads_or(own && fallback < 0);
-    if (any_net) tile_conservative(theta, wbf, feat, bhi, blo, red, o0, dfo);
+    if (any_net) tile_conservative<MI>(theta, wbf, feat, bhi, blo, red, o0, dfo);
     if (!own || fallback >= 0) return;  // exact-force orbits: k_surrogate_fallback
     double phi, gx, gy, gz;
     net_physics(nm, x, y, z, r, o0[t], dfo[t], phi, gx, gy, gz);
@@ -999,6 +1146,12 @@ int check_norm(const gamd_mlp_norm *nm) {
     return GAMD_OK;
 }
 
+// Whether M points go to 16-point tiles (else 32): while every such tile has a
+// compute unit of its own the half-sized tile is done sooner (500 points: 19
+// against 24 us; 4,096: 21 against 24), from there on it reads every weight
+// twice as often (8,192 points: 35 against 27 us).  Same results either way.
+bool tile_points16(size_t M) { return M <= (size_t)cu_count() * 16; }
+
 int check_params(const float *theta, const uint16_t *wbf) {
     return (theta && wbf) ? GAMD_OK : GAMD_ERR_INVALID;
 }
@@ -1044,7 +1197,9 @@ int gamd_mlp_forward(const float *theta, const uint16_t *wbf, const gamd_mlp_nor
     if (check_params(theta, wbf) || check_norm(norm) || (M && (!q || !phi || !grad)))
         return GAMD_ERR_INVALID;
     if (M == 0) return GAMD_OK;
-    hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)((M + CP - 1) / CP)), dim3(256), 0,
+    const bool mi1 = tile_points16(M);
+    hipLaunchKernelGGL(mi1 ? k_mlp_forward<1> : k_mlp_forward<2>,
+                       dim3(grid_for(M, mi1 ? 16 : 32)), dim3(256), 0,
                        as_stream(stream), theta, reinterpret_cast<const __bf16 *>(wbf), *norm, q,
                        (int64_t)M, phi, grad);
     return launch_status();
@@ -1146,7 +1301,9 @@ int gamd_surrogate_leapfrog_step(const float *theta, const uint16_t *wbf, const 
     if (mode != 0 && mode != 1) return GAMD_ERR_INVALID;
     if (N == 0) return GAMD_OK;
     hipStream_t s = as_stream(stream);
-    hipLaunchKernelGGL(k_surrogate_step, dim3((unsigned)((N + CP - 1) / CP)), dim3(256), 0, s,
+    const bool mi1 = tile_points16(N);
+    hipLaunchKernelGGL(mi1 ? k_surrogate_step<1> : k_surrogate_step<2>,
+                       dim3(grid_for(N, mi1 ? 16 : 32)), dim3(256), 0, s,
                        theta, reinterpret_cast<const __bf16 *>(wbf), *norm, w, vsync, E0,
                        fallback_step, w_switch, (int64_t)N, dt, mode, step, tol);
     int rc = launch_status();

@@ -54,6 +54,28 @@ def test_forward_matches_oracle():
     assert np.median(eg) < 1e-4 and eg.max() < 1e-3
 
 
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 33, 4095, 4096, 4097, 8191])
+def test_forward_same_in_every_tile_size(m):
+    """Few points run in 16-point tiles, more in 32-point ones: the same
+    network, the same sums in the same order, so the first m of 20,000 points
+    give the same bits whichever tile they fall into, and match the FP64
+    restatement within the bounds of test_forward_matches_oracle."""
+    from gala_amd import _device as dev
+    sur, pot, S, T = _surrogate(3)
+    q = sur.sample_points(20000, seed=6)
+    phi_a, grad_a = (dev.to_host(a) for a in sur.forward(q))
+    phi, grad = (dev.to_host(a) for a in sur.forward(np.ascontiguousarray(q[:, :m])))
+    np.testing.assert_array_equal(phi, phi_a[:m])
+    np.testing.assert_array_equal(grad, grad_a[:, :m])
+    k = np.unique(np.r_[0:min(m, 40), max(0, m - 40):m])
+    phi_o, grad_o = OM.potential_and_gradient(sur.params().astype(np.float64), q[:, k],
+                                              *_net_args(sur))
+    pb = sur.gm / (np.linalg.norm(q[:, k], axis=0) + sur.rs)
+    assert np.max(np.abs(phi[k] - phi_o) / pb) < 1e-5
+    eg = np.linalg.norm(grad[:, k] - grad_o, axis=0) / np.linalg.norm(grad_o, axis=0)
+    assert eg.max() < 1e-3
+
+
 def test_force_is_the_gradient_of_the_potential():
     """grad Phi_net from the GPU reverse pass equals central finite
     differences of the GPU's own Phi_net: the orbit force is conservative."""
