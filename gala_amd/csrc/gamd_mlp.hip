@@ -22,8 +22,7 @@
 //             orbit force does not use them.
 //
 // Two evaluations of the same network:
-//   * training (tile_forward, k_mlp_forward_train): BF16 activations and
-//     weights, 128-point tiles;
+//   * training (k_train_tile): BF16 activations and weights, 64-point tiles;
 //   * orbits and inference (tile_conservative): the hidden products in
 //     three BF16 matrix-core products, hi*hi + hi*lo + lo*hi of the split
 //     v = hi + lo (hi = bf16(v), lo = bf16(v - hi)), which carries ~16
@@ -33,11 +32,12 @@
 // Matrix-core mapping (gfx950, v_mfma_f32_16x16x32_bf16; operand layout
 // A[i][k] in lane i + 16 (k/8), element k%8; B[k][j] in lane j + 16 (k/8);
 // D[i][j] in lane j + 16 (i/4), element i%4):
-//   * training: a workgroup (4 waves) owns a tile of 128 points; a layer's
-//     activations live in LDS (128 x 256 BF16, rows padded to 264 to keep
-//     the 16-byte fragment reads conflict-free); wave w computes output
-//     units [64w, 64w+64) of all 128 rows: 8 x 4 MFMA tiles, 128 FP32
-//     accumulators per lane;
+//   * a workgroup (4 waves) owns a tile of points; a layer's activations
+//     live in LDS (rows of 256 BF16 padded to 264 to keep the 16-byte fragment
+//     reads conflict-free); wave w computes output units [64w, 64w+64) of all
+//     rows, as the transposed product Z^T = W^T H^T: the weight fragment is
+//     the A operand, so a lane's four accumulators are four consecutive units
+//     of one point (one 8-byte LDS store);
 //   * hidden-layer weights are pre-swizzled into fragment order (and, for
 //     the reverse pass, their transposes), so each wave reads 1 KB
 //     contiguous per (16-unit tile, K step) from L2.
@@ -54,7 +54,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int H = 256;        // hidden width
-constexpr int TILE = 128;     // points per workgroup
 constexpr int LDSR = 264;     // padded LDS row (BF16 elements)
 // flat FP32 parameter layout
 constexpr int OFF_W1 = 0, OFF_B1 = OFF_W1 + 4 * H;
@@ -64,12 +63,10 @@ constexpr int OFF_W4 = OFF_B3 + H, OFF_B4 = OFF_W4 + H * H;
 constexpr int OFF_W5 = OFF_B4 + H, OFF_B5 = OFF_W5 + H * 4;
 constexpr int NPARAM = OFF_B5 + 4;  // 199,684
 // BF16 copies of W2..W4, each block 3 H^2 (one H^2 per layer): fragment
-// order (hi), row-major (hi, for the training backward), fragment order of
-// the low parts, and fragment order of the transposes (hi, then lo) for the
-// reverse pass of tile_conservative
-constexpr int BF_SW = 0, BF_ROW = 3 * H * H, BF_SWLO = 6 * H * H, BF_TSW = 9 * H * H,
-              BF_TSWLO = 12 * H * H;
-constexpr int NBF = 15 * H * H;
+// order of the high and the low parts, and of the transposes (high, low) for
+// the reverse passes
+constexpr int BF_SW = 0, BF_SWLO = 3 * H * H, BF_TSW = 6 * H * H, BF_TSWLO = 9 * H * H;
+constexpr int NBF = 12 * H * H;
 
 // logistic function from the hardware exp2 and reciprocal (v_exp_f32,
 // v_rcp_f32, ~1 ulp each): the activations are rounded to BF16 (8 bits)
@@ -138,121 +135,6 @@ __device__ __forceinline__ void net_physics(const gamd_mlp_norm &nm, double x, d
     gy = a * y + b * oy;
     gz = a * z + b * oz;
 }
-
-// ---------------------------------------------------------------------------
-// fused forward of one 128-point tile.  feat: LDS [TILE][4]; on return the
-// raw outputs are in LDS out[TILE][4].  With TRAIN, pre-activations and
-// activations of the four hidden layers go to global (BF16, [4][M][256]).
-template <bool TRAIN>
-__device__ __forceinline__ void tile_forward(const float *__restrict__ theta, const __bf16 *__restrict__ wsw,
-                             const float (*feat)[4], __bf16 *buf, float (*out)[4],
-                             int64_t row0, int64_t M, __bf16 *__restrict__ Zs,
-                             __bf16 *__restrict__ Hs) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    // layer 1: 4 -> 256 in FP32; thread t owns unit j = t
-    {
-        const int j = t;
-        const float w0 = theta[OFF_W1 + 0 * H + j], w1 = theta[OFF_W1 + 1 * H + j];
-        const float w2 = theta[OFF_W1 + 2 * H + j], w3 = theta[OFF_W1 + 3 * H + j];
-        const float bj = theta[OFF_B1 + j];
-#pragma unroll 4
-        for (int p = 0; p < TILE; p++) {
-            const float z = bj + feat[p][0] * w0 + feat[p][1] * w1 + feat[p][2] * w2 + feat[p][3] * w3;
-            const float h = silu(z);
-            buf[p * LDSR + j] = tobf(h);
-            if (TRAIN && row0 + p < M) {
-                Zs[(0 * M + row0 + p) * H + j] = tobf(z);
-                Hs[(0 * M + row0 + p) * H + j] = tobf(h);
-            }
-        }
-    }
-    __syncthreads();
-    // layers 2..4 on the matrix cores
-    // one activation buffer: every wave holds its 64 units of the whole
-    // layer in accumulators, so the layer reads the buffer, waits for every
-    // wave, then overwrites it (68 KB of LDS: two workgroups per CU, whose
-    // matrix-core and SiLU phases overlap)
-#pragma unroll 1
-    for (int l = 0; l < 3; l++) {
-        const float *bias = theta + (l == 0 ? OFF_B2 : l == 1 ? OFF_B3 : OFF_B4);
-        const __bf16 *W = wsw + (size_t)l * H * H;
-        // the wave's 64 units in one pass (128 FP32 accumulators per lane):
-        // each activation fragment is read from LDS once per layer
-        {
-            constexpr int NT = 4;  // 16-unit tiles per wave
-            f32x4 acc[8][NT];
-#pragma unroll
-            for (int mi = 0; mi < 8; mi++)
-#pragma unroll
-                for (int ni = 0; ni < NT; ni++) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-            for (int ks = 0; ks < 8; ks++) {
-                bf16x8 b[NT];
-#pragma unroll
-                for (int ni = 0; ni < NT; ni++)
-                    b[ni] = *reinterpret_cast<const bf16x8 *>(
-                        W + (((4 * w + ni) * 8 + ks) * 64 + lane) * 8);
-#pragma unroll
-                for (int mi = 0; mi < 8; mi++) {
-                    const bf16x8 a = *reinterpret_cast<const bf16x8 *>(
-                        buf + (16 * mi + (lane & 15)) * LDSR + 32 * ks + 8 * (lane >> 4));
-                    // the transposed product, Z^T = W^T H^T: the weight fragment
-                    // is the A operand and the activations the B operand, so a
-                    // lane's four accumulators are four consecutive units of
-                    // one point (one 8-byte store below instead of four 2-byte)
-#pragma unroll
-                    for (int ni = 0; ni < NT; ni++)
-                        acc[mi][ni] =
-                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[ni], a, acc[mi][ni], 0, 0, 0);
-                }
-            }
-            __syncthreads();  // every wave has read the layer's input
-#pragma unroll
-            for (int mi = 0; mi < 8; mi++)
-#pragma unroll
-                for (int ni = 0; ni < NT; ni++) {
-                    const int unit = 64 * w + 16 * ni + 4 * (lane >> 4);
-                    const int row = 16 * mi + (lane & 15);
-                    const f32x4 bc = *reinterpret_cast<const f32x4 *>(bias + unit);
-                    __bf16 hv[4], zv[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float z = acc[mi][ni][e] + bc[e];
-                        hv[e] = tobf(silu(z));
-                        zv[e] = tobf(z);
-                    }
-                    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-                    *reinterpret_cast<bf16x4 *>(buf + row * LDSR + unit) =
-                        bf16x4{hv[0], hv[1], hv[2], hv[3]};
-                    if (TRAIN && row0 + row < M) {
-                        *reinterpret_cast<bf16x4 *>(Zs + ((size_t)(l + 1) * M + row0 + row) * H + unit) =
-                            bf16x4{zv[0], zv[1], zv[2], zv[3]};
-                        *reinterpret_cast<bf16x4 *>(Hs + ((size_t)(l + 1) * M + row0 + row) * H + unit) =
-                            bf16x4{hv[0], hv[1], hv[2], hv[3]};
-                    }
-                }
-        }
-        __syncthreads();
-    }
-    // layer 5: 256 -> 4 in FP32 from the BF16 activations; thread t: point
-    // t/2, outputs 2(t%2), 2(t%2)+1
-    {
-        const int p = t >> 1, o0 = 2 * (t & 1);
-        float s0 = theta[OFF_B5 + o0], s1 = theta[OFF_B5 + o0 + 1];
-        const __bf16 *hrow = buf + p * LDSR;
-#pragma unroll 8
-        for (int j = 0; j < H; j++) {
-            const float hj = frombf(hrow[j]);
-            s0 += hj * theta[OFF_W5 + j * 4 + o0];
-            s1 += hj * theta[OFF_W5 + j * 4 + o0 + 1];
-        }
-        out[p][o0] = s0;
-        out[p][o0 + 1] = s1;
-    }
-    __syncthreads();
-}
-
-constexpr int LDS_BYTES = TILE * LDSR * 2;
 
 // ---------------------------------------------------------------------------
 // The precise evaluation of one tile of CP = 16 MI points: o0 and d o0 / d f
@@ -620,332 +502,524 @@ __global__ __launch_bounds__(256, 2) void k_mlp_forward(const float *__restrict_
     }
 }
 
-// training forward: feat (M,4) FP32 -> Zs, Hs (BF16 [4][M][256]), Y (M,4)
-__global__ __launch_bounds__(256, 2) void k_mlp_forward_train(const float *__restrict__ theta,
-                                                           const __bf16 *__restrict__ wsw,
-                                                           const float *__restrict__ featg,
-                                                           int64_t M, __bf16 *__restrict__ Zs,
-                                                           __bf16 *__restrict__ Hs,
-                                                           float *__restrict__ Y) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __bf16 *buf = reinterpret_cast<__bf16 *>(smem);
-    __shared__ float feat[TILE][4];
-    __shared__ float out[TILE][4];
-    const int t = threadIdx.x;
-    const int64_t row0 = (int64_t)blockIdx.x * TILE;
-    if (t < TILE) {
-        const int64_t i = row0 + t;
-#pragma unroll
-        for (int c = 0; c < 4; c++) feat[t][c] = i < M ? featg[i * 4 + c] : 0.0f;
-    }
-    __syncthreads();
-    tile_forward<true>(theta, wsw, feat, buf, out, row0, M, Zs, Hs);
-    if (t < TILE && row0 + t < M)
-#pragma unroll
-        for (int c = 0; c < 4; c++) Y[(row0 + t) * 4 + c] = out[t][c];
-}
-
 // ---------------------------------------------------------------------------
-// generic BF16 GEMM on the matrix cores for the backward pass:
-//   C[m][n] = sum_k A[m][k] B[k][n], A[m][k] = A[m*sam + k*sak], B[k][n] = B[k*sbk + n*sbn]
-// EPI 0: C (FP32, ldc) = acc.  EPI 1: out (BF16, ldc) = acc * silu'(Zprev[m][n]).
-// Tile 64 x 64 per workgroup (4 waves of 32 x 32); M, N multiples of 64, K of 32.
-// KC: both operands contiguous along k (sak = sbk = 1), read as 16-byte vectors.
-template <int EPI, bool KC = false>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const __bf16 *__restrict__ A,
-                                              int64_t sam, int64_t sak,
-                                              const __bf16 *__restrict__ B, int64_t sbk,
-                                              int64_t sbn, float *__restrict__ C,
-                                              __bf16 *__restrict__ Cb, int64_t ldc,
-                                              const __bf16 *__restrict__ Zprev) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int m0 = blockIdx.x * 64 + 32 * (w >> 1);
-    const int n0 = blockIdx.y * 64 + 32 * (w & 1);
-    f32x4 acc[2][2];
+// Training: loss, its gradient and Adam.
+//
+// k_train_tile takes 64 points through the network and back: the four hidden
+// layers, the output, the loss and the error signals dZ_4 .. dZ_1, with BF16
+// weights and activations and FP32 accumulation.  Wave w owns units
+// [64w, 64w + 64) of every layer both ways, so the pre-activations it needs
+// for the SiLU derivatives stay in its registers (BF16); the activations
+// H_1 .. H_3 and the error signals dZ_2 .. dZ_4 that the hidden weights'
+// gradients need go to memory, once each; every sum over the tile's points
+// (first and output layers' weights, biases, loss) is finished in the tile
+// and leaves as one row of 3,080 partial sums.
+//
+// k_wgrad forms the three hidden weight gradients H_{l-1}^T dZ_l, split over
+// slices of the points into partial matrices; k_grad_reduce adds slices and
+// tile rows in a fixed order, so gradients are the same in every run.
+//
+// 32,768 points: k_train_tile 61 us, k_wgrad 27, k_grad_reduce 9 and Adam 6;
+// 104 us per step end to end.  The same step took 450 us as twenty launches:
+// a forward pass that wrote every pre-activation and activation (134 MB), a
+// product per layer that read them back, and reductions over the points by
+// atomic adds from every block (50 us per weight gradient, 31 us for dW5).
+// k_train_tile is bound by its vector work (~5,500 instructions and 768
+// exp2/rcp per wave, two waves per SIMD) beside 100 MB of stores; k_wgrad and
+// k_grad_reduce by their 180 and 39 MB.  64-point tiles of four waves let two
+// workgroups share a compute unit, one's products behind the other's SiLU.
+
+constexpr int TP = 64;  // points per workgroup of k_train_tile
+// one tile's partial sums: dW1 [4][256], db1..db4 [4][256], dW5 [256][4], db5, loss
+constexpr int PT_W1 = 0, PT_B = 4 * H, PT_W5 = 8 * H, PT_B5 = 12 * H, PT_LOSS = PT_B5 + 4;
+constexpr int PT_N = 12 * H + 8;
+
+// one K step of a wave's weight fragments (high parts only)
+__device__ __forceinline__ void load_frags_hi(bf16x8 (&f)[4], const NetBufs &nb, unsigned hi,
+                                              int ks) {
+    const unsigned lane = threadIdx.x & 63, w = wave_id();
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int li = lane & 15, lk = 8 * (lane >> 4);
-    // split-K over gridDim.z (each slice a multiple of 32; EPI 0 then adds)
-    const int kslice = K / (int)gridDim.z;
-    const int k_lo = (int)blockIdx.z * kslice, k_hi = k_lo + kslice;
-    for (int k0 = k_lo; k0 < k_hi; k0 += 32) {
-        bf16x8 a[2], b[2];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int64_t row = m0 + 16 * i + li;
-            if (KC) {
-                a[i] = *reinterpret_cast<const bf16x8 *>(A + row * sam + k0 + lk);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) a[i][e] = A[row * sam + (int64_t)(k0 + lk + e) * sak];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int64_t col = n0 + 16 * j + li;
-            if (KC) {
-                b[j] = *reinterpret_cast<const bf16x8 *>(B + k0 + lk + col * sbn);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) b[j][e] = B[(int64_t)(k0 + lk + e) * sbk + col * sbn];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned o = ((4 * w + ni) * 8 + ks) * 64 * 8;
+        f[ni] = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(nb.w, lane * 16, (hi + o) * 2, 0));
     }
+}
+
+// acc = weights (fragment order at element offset hi) times the 64 points in
+// buf; weights one step ahead as in split_layer (f[0] holds the first step on
+// entry and the next block's on return)
+template <bool NEXT>
+__device__ __forceinline__ void train_layer(const NetBufs &nb, unsigned hi, unsigned nhi,
+                                            const __bf16 *buf, bf16x8 (&f)[2][4],
+                                            f32x4 (&acc)[4][4]) {
+    const unsigned lane = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int mi = 0; mi < 4; mi++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int ni = 0; ni < 4; ni++) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 8; ks++) {
+        if (ks < 7)
+            load_frags_hi(f[(ks + 1) & 1], nb, hi, ks + 1);
+        else if (NEXT)
+            load_frags_hi(f[0], nb, nhi, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        bf16x8 a[4];
+#pragma unroll
+        for (int mi = 0; mi < 4; mi++)
+            a[mi] = *reinterpret_cast<const bf16x8 *>(buf + (16 * mi + (lane & 15)) * LDSR +
+                                                      32 * ks + 8 * (lane >> 4));
+#pragma unroll
+        for (int mi = 0; mi < 4; mi++)
+#pragma unroll
+            for (int ni = 0; ni < 4; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ks & 1][ni], a[mi],
+                                                                      acc[mi][ni], 0, 0, 0);
+    }
+}
+
+// the tile's (64, 256) layer in buf to its rows at dst of a (M, 256) matrix,
+// 16 bytes per thread and step (through a descriptor of those rows: one
+// 32-bit offset serves all steps)
+__device__ __forceinline__ void store_tile(const __bf16 *buf, __bf16 *__restrict__ dst) {
+    const unsigned t = threadIdx.x;
+    const __amdgpu_buffer_rsrc_t out =
+        __builtin_amdgcn_make_buffer_rsrc(dst, 0, TP * H * 2, 0x00027000);
+    const __bf16 *src = buf + (t >> 5) * LDSR + 8 * (t & 31);
+#pragma unroll
+    for (int k = 0; k < TP / 8; k++) {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(src + 8 * k * LDSR);
+        __builtin_amdgcn_raw_buffer_store_b128(v, out, t * 16, k * 8 * H * 2, 0);
+        if (k & 1) __builtin_amdgcn_sched_barrier(0);  // two in flight: registers are scarce
+    }
+}
+
+// four BF16 values in two registers.  The empty asm makes the pair opaque:
+// otherwise each half travels in a register of its own, 64 per layer too many
+struct Packed4 {
+    unsigned v[2];
+    __device__ __forceinline__ void set(const bf16x4 &x) {
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 u = __builtin_bit_cast(u32x2, x);
+        v[0] = u[0];
+        v[1] = u[1];
+        asm("" : "+v"(v[0]), "+v"(v[1]));
+    }
+    // element e as FP32 (a BF16 value is the top half of its FP32 form)
+    __device__ __forceinline__ float get(int e) const {
+        const unsigned u = v[e >> 1];
+        return __builtin_bit_cast(float, e & 1 ? u & 0xffff0000u : u << 16);
+    }
+};
+
+// z = acc + bias (BF16 copies kept in z) and silu(z) into buf
+template <int L>
+__device__ __forceinline__ void train_forward_epilogue(const NetBufs &nb, const f32x4 (&acc)[4][4],
+                                                       __bf16 *buf, Packed4 (&z)[4][4]) {
+    const unsigned lane = threadIdx.x & 63, w = wave_id(), lu = 4 * (lane >> 4);
+    constexpr unsigned bias = L == 2 ? OFF_B2 : L == 3 ? OFF_B3 : OFF_B4;
+#pragma unroll
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned tile = 64 * w + 16 * ni;
+        const f32x4 bc = theta4(nb, bias + tile, lu);
+#pragma unroll
+        for (int mi = 0; mi < 4; mi++) {
+            bf16x4 hv, zv;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int64_t row = m0 + 16 * i + 4 * (lane >> 4) + e;
-                const int64_t col = n0 + 16 * j + li;
-                if (EPI == 0) {
-                    if (gridDim.z > 1)
-                        atomicAdd(&C[row * ldc + col], acc[i][j][e]);
-                    else
-                        C[row * ldc + col] = acc[i][j][e];
-                } else
-                    Cb[row * ldc + col] = tobf(acc[i][j][e] * dsilu(frombf(Zprev[row * ldc + col])));
+                const float v = acc[mi][ni][e] + bc[e];
+                hv[e] = tobf(silu(v));
+                zv[e] = tobf(v);
             }
-}
-
-// Weight gradient of a hidden layer, C[m][n] += sum_p A[p][m] B[p][n] over
-// this workgroup's slice of the P points (split over gridDim.z), with A and B
-// row-major [P][256] BF16 (a layer's input activations and its pre-activation
-// gradients) and C [256][256] FP32 (atomic adds across slices; the caller
-// zeroes it).  The reduction runs along the points, which both operands store
-// 512 bytes apart, so tiles of 64 points x 64 columns are read with coalesced
-// 16-byte loads and written transposed into LDS: each matrix-core fragment (8
-// consecutive points of one column) is then one 16-byte LDS read.  64 x 64
-// outputs per workgroup, a 32 x 32 quarter per wave.  With gb, the
-// workgroups of the first row tile also add the column sums of B (the bias
-// gradient) into gb from the tiles they stage.
-constexpr int WG_KC = 64;          // points per LDS stage
-constexpr int WG_LDK = WG_KC + 8;  // padded LDS row in BF16 (144 bytes, 16-byte aligned)
-
-__global__ __launch_bounds__(256) void k_wgrad(int P, const __bf16 *__restrict__ A,
-                                               const __bf16 *__restrict__ B,
-                                               float *__restrict__ C, float *__restrict__ gb) {
-    __shared__ __align__(16) __bf16 As[64][WG_LDK];
-    __shared__ __align__(16) __bf16 Bs[64][WG_LDK];
-    __shared__ float red[4][64];
-    const bool colsum = gb != nullptr && blockIdx.x == 0;  // uniform over the workgroup
-    float cs = 0.f;  // column t % 64, points 16 (t / 64) .. + 15 of each stage
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int mt = blockIdx.x * 64, nt = blockIdx.y * 64;  // the workgroup's output tile
-    const int mw = 32 * (w >> 1), nw = 32 * (w & 1);       // the wave's quarter of it
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int li = lane & 15, lk = 8 * (lane >> 4);
-    const int pslice = P / (int)gridDim.z;
-    const int p_lo = (int)blockIdx.z * pslice, p_hi = p_lo + pslice;
-    // staging: thread t loads points r and r + 32 of the stage, columns c8 .. c8 + 7
-    const int r = t >> 3, c8 = 8 * (t & 7);
-    for (int p0 = p_lo; p0 < p_hi; p0 += WG_KC) {
-        bf16x8 va[2], vb[2];
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
-            const int64_t p = (int64_t)p0 + r + 32 * hh;
-            va[hh] = *reinterpret_cast<const bf16x8 *>(A + p * H + mt + c8);
-            vb[hh] = *reinterpret_cast<const bf16x8 *>(B + p * H + nt + c8);
-        }
-        __syncthreads();  // every wave has read the previous stage
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                As[c8 + e][r + 32 * hh] = va[hh][e];
-                Bs[c8 + e][r + 32 * hh] = vb[hh][e];
-            }
-        __syncthreads();
-        if (colsum) {
-            const bf16x8 *src = reinterpret_cast<const bf16x8 *>(&Bs[t & 63][16 * (t >> 6)]);
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const bf16x8 v = src[q];
-#pragma unroll
-                for (int e = 0; e < 8; e++) cs += frombf(v[e]);
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < WG_KC; ks += 32) {
-            bf16x8 a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                a[i] = *reinterpret_cast<const bf16x8 *>(&As[mw + 16 * i + li][ks + lk]);
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                b[j] = *reinterpret_cast<const bf16x8 *>(&Bs[nw + 16 * j + li][ks + lk]);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            z[mi][ni].set(zv);
+            *reinterpret_cast<bf16x4 *>(buf + (16 * mi + (lane & 15)) * LDSR + tile + lu) = hv;
         }
     }
+}
+
+// sum over the 16 lanes (one DPP row) that hold one unit's points, in every
+// lane: rotations by 8, 4, 2 and 1 inside the row, no LDS traffic
+template <int N>
+__device__ __forceinline__ float row_ror(float v) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float sum16(float v) {
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    v += row_ror<1>(v);
+    return v;
+}
+
+// dZ = (W^T dZ_next) silu'(z) into buf, its sums over the tile's points to gb
+__device__ __forceinline__ void train_reverse_epilogue(const f32x4 (&acc)[4][4],
+                                                       const Packed4 (&z)[4][4], __bf16 *buf,
+                                                       float *__restrict__ gb) {
+    const unsigned lane = threadIdx.x & 63, w = wave_id(), lu = 4 * (lane >> 4);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned unit = 64 * w + 16 * ni + lu;
+        f32x4 cs = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int mi = 0; mi < 4; mi++) {
+            bf16x4 d;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int row = mt + mw + 16 * i + 4 * (lane >> 4) + e;
-                const int col = nt + nw + 16 * j + li;
-                atomicAdd(&C[row * H + col], acc[i][j][e]);
+                d[e] = tobf(acc[mi][ni][e] * dsilu(z[mi][ni].get(e)));
+                cs[e] += frombf(d[e]);
             }
-    if (colsum) {
-        red[t >> 6][t & 63] = cs;
-        __syncthreads();
-        if (t < 64) atomicAdd(&gb[nt + t], red[0][t] + red[1][t] + red[2][t] + red[3][t]);
+            *reinterpret_cast<bf16x4 *>(buf + (16 * mi + (lane & 15)) * LDSR + unit) = d;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) cs[e] = sum16(cs[e]);
+        if ((lane & 15) == 0) *reinterpret_cast<f32x4 *>(gb + unit) = cs;
     }
 }
 
-// loss and dY = 2 (Y - T) / M; per-block partial loss sums
-__global__ void k_loss(const float *__restrict__ Y, const float *__restrict__ T, int64_t M,
-                       float *__restrict__ dY, float *__restrict__ partial) {
-    __shared__ float red[256];
+__global__ __launch_bounds__(256, 2) void k_train_tile(
+    const float *__restrict__ theta, const __bf16 *__restrict__ wbf,
+    const float *__restrict__ featg, const float *__restrict__ targetg, int64_t M,
+    __bf16 *__restrict__ Hs, __bf16 *__restrict__ Ds, float *__restrict__ part) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) __bf16 buf[TP * LDSR];
+    __shared__ __align__(16) float fs[TP][4];   // features
+    __shared__ __align__(16) float dy[TP][4];   // d loss / d output
+    __shared__ __align__(16) float w5t[4][H];   // output weights, transposed
+    __shared__ __align__(16) float half[H][4];  // dW5 of the second half of the points
+    __shared__ float red[4];
+    const unsigned t = threadIdx.x, lane = t & 63, w = wave_id(), lu = 4 * (lane >> 4);
+    const int64_t row0 = (int64_t)blockIdx.x * TP;
+    const NetBufs nb = net_bufs(theta, wbf);
+    constexpr unsigned LW = H * H;
+    const size_t layer = (size_t)M * H;
+    __bf16 *Ht = Hs + row0 * H, *Dt = Ds + row0 * H;
+    float *pt = part + (size_t)blockIdx.x * PT_N;
+    bf16x8 f[2][4];
+    load_frags_hi(f[0], nb, BF_SW, 0);
+    fs[t >> 2][t & 3] = featg[row0 * 4 + t];
+    const float target = targetg[row0 * 4 + t];
+    {
+        const f32x4 r = theta4(nb, OFF_W5, 4 * t);
+#pragma unroll
+        for (int o = 0; o < 4; o++) w5t[o][t] = r[o];
+    }
+    __syncthreads();
+    // layer 1: 4 -> 256 in FP32, two units of half of the points per thread
+    {
+        const unsigned j = 2 * (t & 127), p0 = (t >> 7) * (TP / 2);
+        const f32x2 w0 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 0 * H + j);
+        const f32x2 w1 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 1 * H + j);
+        const f32x2 w2 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 2 * H + j);
+        const f32x2 w3 = *reinterpret_cast<const f32x2 *>(theta + OFF_W1 + 3 * H + j);
+        const f32x2 bj = *reinterpret_cast<const f32x2 *>(theta + OFF_B1 + j);
+#pragma unroll 4
+        for (unsigned p = p0; p < p0 + TP / 2; p++) {
+            const f32x4 fp = *reinterpret_cast<const f32x4 *>(fs[p]);
+            bf16x2 hv;
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                hv[e] = tobf(silu(bj[e] + fp[0] * w0[e] + fp[1] * w1[e] + fp[2] * w2[e] + fp[3] * w3[e]));
+            *reinterpret_cast<bf16x2 *>(buf + p * LDSR + j) = hv;
+        }
+    }
+    __syncthreads();
+    f32x4 acc[4][4];
+    Packed4 z2[4][4], z3[4][4], z4[4][4];
+    store_tile(buf, Ht);
+    train_layer<true>(nb, BF_SW, BF_SW + LW, buf, f, acc);
+    __syncthreads();
+    train_forward_epilogue<2>(nb, acc, buf, z2);
+    __syncthreads();
+    store_tile(buf, Ht + layer);
+    train_layer<true>(nb, BF_SW + LW, BF_SW + 2 * LW, buf, f, acc);
+    __syncthreads();
+    train_forward_epilogue<3>(nb, acc, buf, z3);
+    __syncthreads();
+    store_tile(buf, Ht + 2 * layer);
+    train_layer<true>(nb, BF_SW + 2 * LW, BF_TSW + 2 * LW, buf, f, acc);
+    __syncthreads();
+    train_forward_epilogue<4>(nb, acc, buf, z4);
+    __syncthreads();
+    // output, loss and dY: thread t holds output t % 4 of point t / 4
+    {
+        const unsigned p = t >> 2, o = t & 3;
+        float y = theta[OFF_B5 + o];
+        const __bf16 *hrow = buf + p * LDSR;
+#pragma unroll 4
+        for (int j = 0; j < H; j += 8) {
+            const bf16x8 h = *reinterpret_cast<const bf16x8 *>(hrow + j);
+            const f32x4 wa = *reinterpret_cast<const f32x4 *>(&w5t[o][j]);
+            const f32x4 wb = *reinterpret_cast<const f32x4 *>(&w5t[o][j + 4]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) y += frombf(h[e]) * wa[e];
+#pragma unroll
+            for (int e = 0; e < 4; e++) y += frombf(h[4 + e]) * wb[e];
+        }
+        const float d = y - target;
+        const float g = 2.0f * d / (float)M;
+        dy[p][o] = g;
+        float l = d * d, gs = g;
+#pragma unroll
+        for (int m = 4; m < 64; m <<= 1) gs += __shfl_xor(gs, m);
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) l += __shfl_xor(l, m);
+        // db5 and the loss: this wave's sixteen points, then the four waves
+        if (lane < 4) half[w][lane] = gs;
+        if (lane == 0) red[w] = l;
+    }
+    __syncthreads();
+    if (t < 4) pt[PT_B5 + t] = half[0][t] + half[1][t] + half[2][t] + half[3][t];
+    if (t == 4) pt[PT_LOSS] = red[0] + red[1] + red[2] + red[3];
+    __syncthreads();
+    // dW5: units j, j + 1 over half of the points, the halves joined in LDS
+    {
+        const unsigned j = 2 * (t & 127), p0 = (t >> 7) * (TP / 2);
+        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (unsigned p = p0; p < p0 + TP / 2; p++) {
+            const bf16x2 h = *reinterpret_cast<const bf16x2 *>(buf + p * LDSR + j);
+            const f32x4 g = *reinterpret_cast<const f32x4 *>(dy[p]);
+            const float h0 = frombf(h[0]), h1 = frombf(h[1]);
+#pragma unroll
+            for (int o = 0; o < 4; o++) {
+                s0[o] += h0 * g[o];
+                s1[o] += h1 * g[o];
+            }
+        }
+        if (t >= 128) {
+            *reinterpret_cast<f32x4 *>(half[j]) = s0;
+            *reinterpret_cast<f32x4 *>(half[j + 1]) = s1;
+        }
+        __syncthreads();  // the layer's last readers too: dZ4 overwrites it below
+        if (t < 128) {
+            *reinterpret_cast<f32x4 *>(pt + PT_W5 + 4 * j) = s0 + *reinterpret_cast<const f32x4 *>(half[j]);
+            *reinterpret_cast<f32x4 *>(pt + PT_W5 + 4 * j + 4) =
+                s1 + *reinterpret_cast<const f32x4 *>(half[j + 1]);
+        }
+    }
+    // dZ4 = (dY W5^T) silu'(z4)
+#pragma unroll
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned tile = 64 * w + 16 * ni;
+        f32x4 w5[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) w5[e] = theta4(nb, OFF_W5 + 4 * (tile + e), 4 * lu);
+#pragma unroll
+        for (int mi = 0; mi < 4; mi++) {
+            const f32x4 g = *reinterpret_cast<const f32x4 *>(dy[16 * mi + (lane & 15)]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float s = 0.f;
+#pragma unroll
+                for (int o = 0; o < 4; o++) s += g[o] * w5[e][o];
+                acc[mi][ni][e] = s;
+            }
+        }
+    }
+    train_reverse_epilogue(acc, z4, buf, pt + PT_B + 3 * H);
+    __syncthreads();
+    store_tile(buf, Dt + 2 * layer);
+    train_layer<true>(nb, BF_TSW + 2 * LW, BF_TSW + LW, buf, f, acc);
+    __syncthreads();
+    train_reverse_epilogue(acc, z3, buf, pt + PT_B + 2 * H);
+    __syncthreads();
+    store_tile(buf, Dt + layer);
+    train_layer<true>(nb, BF_TSW + LW, BF_TSW, buf, f, acc);
+    __syncthreads();
+    train_reverse_epilogue(acc, z2, buf, pt + PT_B + H);
+    __syncthreads();
+    store_tile(buf, Dt);
+    train_layer<false>(nb, BF_TSW, 0, buf, f, acc);
+    // layer 1: its pre-activations recomputed, dW1 and db1 summed over the tile
+    f32x4 fr[4];
+#pragma unroll
+    for (int mi = 0; mi < 4; mi++) fr[mi] = *reinterpret_cast<const f32x4 *>(fs[16 * mi + (lane & 15)]);
+#pragma unroll
+    for (int ni = 0; ni < 4; ni++) {
+        const unsigned tile = 64 * w + 16 * ni;
+        f32x4 w1[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) w1[c] = theta4(nb, OFF_W1 + c * H + tile, lu);
+        const f32x4 b1 = theta4(nb, OFF_B1 + tile, lu);
+        f32x4 cs = {0.f, 0.f, 0.f, 0.f}, gw[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) gw[c] = cs;
+#pragma unroll
+        for (int mi = 0; mi < 4; mi++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float z = b1[e] + fr[mi][0] * w1[0][e] + fr[mi][1] * w1[1][e] +
+                                fr[mi][2] * w1[2][e] + fr[mi][3] * w1[3][e];
+                const float d = frombf(tobf(acc[mi][ni][e] * dsilu(frombf(tobf(z)))));
+                cs[e] += d;
+#pragma unroll
+                for (int c = 0; c < 4; c++) gw[c][e] += fr[mi][c] * d;
+            }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            cs[e] = sum16(cs[e]);
+#pragma unroll
+            for (int c = 0; c < 4; c++) gw[c][e] = sum16(gw[c][e]);
+        }
+        if ((lane & 15) == 0) {
+            *reinterpret_cast<f32x4 *>(pt + PT_B + tile + lu) = cs;
+#pragma unroll
+            for (int c = 0; c < 4; c++) *reinterpret_cast<f32x4 *>(pt + PT_W1 + c * H + tile + lu) = gw[c];
+        }
+    }
+}
+
+// Hidden weight gradients: layer l's (256, 256) matrix H_l^T dZ_l over one
+// slice of the points, into that slice's partial matrix.  A workgroup of 8
+// waves forms 256 inputs x 128 outputs, 64 x 64 per wave.  Both operands are
+// stored point by point while the products run along the points: 64-point
+// stages go through LDS as they are stored (the next stage's reads in flight
+// in registers meanwhile) and come out transposed (ds_read_b64_tr_b16: four
+// points of one unit per lane).  Rows are padded by 32 bytes, which spreads
+// the 16 rows of a transposed read over all banks.
+constexpr int WG_P = 64;                            // points per stage
+constexpr int WG_SLICES = 42;                       // 3 layers x 2 halves x 42: one round of 256 CUs
+constexpr int WG_LA = H + 16, WG_LB = H / 2 + 16;   // LDS row lengths
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bf16x8 tr_frag(const __bf16 *lds, unsigned row, unsigned row_len,
+                                          unsigned col) {
+    typedef __attribute__((address_space(3))) s16x4 lds_v;
+    const unsigned li = threadIdx.x & 15;
+    const __bf16 *p = lds + (row + (li >> 2)) * row_len + col + 4 * (li & 3);
+    struct {
+        s16x4 lo, hi;
+    } v;
+    v.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v *)p);
+    v.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v *)(p + 4 * row_len));
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+// stages [lo, hi) of slice s of n
+__host__ __device__ __forceinline__ int slice_begin(int stages, int slices, int s) {
+    return (int)((int64_t)stages * s / slices);
+}
+
+__global__ __launch_bounds__(512, 2) void k_wgrad(int64_t M, int slices,
+                                                  const __bf16 *__restrict__ Hs,
+                                                  const __bf16 *__restrict__ Ds,
+                                                  float *__restrict__ part) {
+    __shared__ __align__(16) __bf16 As[WG_P * WG_LA];
+    __shared__ __align__(16) __bf16 Bs[WG_P * WG_LB];
+    // consecutive workgroups go to the 8 XCDs in turn: the two halves of one
+    // (slice, layer) are 8 apart, so they share their reads of H in one L2
+    const unsigned half = (blockIdx.x >> 3) & 1, u = (blockIdx.x & 7) + 8 * (blockIdx.x >> 4);
+    if (u >= 3u * slices) return;
+    const unsigned l = u % 3, s = u / 3;
+    const unsigned t = threadIdx.x, lane = t & 63, w = wave_id();
+    const int64_t off = (int64_t)l * M * H;
+    const int stages = (int)(M / WG_P);
+    const int lo = slice_begin(stages, slices, s), hi = slice_begin(stages, slices, s + 1);
+    const __bf16 *A = Hs + off, *B = Ds + off + half * (H / 2);
+    bf16x8 ra[4], rb[2];
+    auto fetch = [&](int st) {
+        const int64_t p0 = (int64_t)st * WG_P;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            ra[k] = *reinterpret_cast<const bf16x8 *>(A + (p0 + 16 * k + (t >> 5)) * H + 8 * (t & 31));
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            rb[k] = *reinterpret_cast<const bf16x8 *>(B + (p0 + 32 * k + (t >> 4)) * H + 8 * (t & 15));
+    };
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned mw = 64 * (w >> 1), nw = 64 * (w & 1);
+    if (lo < hi) fetch(lo);
+    for (int st = lo; st < hi; st++) {
+        __syncthreads();  // the previous stage has been read
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            *reinterpret_cast<bf16x8 *>(As + (16 * k + (t >> 5)) * WG_LA + 8 * (t & 31)) = ra[k];
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            *reinterpret_cast<bf16x8 *>(Bs + (32 * k + (t >> 4)) * WG_LB + 8 * (t & 15)) = rb[k];
+        __syncthreads();
+        if (st + 1 < hi) fetch(st + 1);
+#pragma unroll
+        for (int ks = 0; ks < WG_P; ks += 32) {
+            const unsigned row = ks + 8 * (lane >> 4);
+            bf16x8 a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[i] = tr_frag(As, row, WG_LA, mw + 16 * i);
+#pragma unroll
+            for (int j = 0; j < 4; j++) b[j] = tr_frag(Bs, row, WG_LB, nw + 16 * j);
+            // outputs as the A operand: a lane's four sums are four
+            // consecutive outputs of one input (one 16-byte store below)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+        }
+    }
+    float *out = part + ((size_t)s * 3 + l) * H * H + half * (H / 2);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            *reinterpret_cast<f32x4 *>(out + (mw + 16 * i + (lane & 15)) * H + nw + 16 * j +
+                                       4 * (lane >> 4)) = acc[i][j];
+}
+
+// Gradients from the partial sums: blocks [0, RW) four hidden weights per
+// thread over the slices, the others 32 columns of the tiles' rows each (8
+// row groups, joined in LDS).
+constexpr int RW = 3 * H * H / 1024, RP = (PT_N + 31) / 32;
+
+__global__ __launch_bounds__(256) void k_grad_reduce(const float *__restrict__ wpart, int slices,
+                                                     const float *__restrict__ tpart, int tiles,
+                                                     float *__restrict__ grad,
+                                                     float *__restrict__ loss) {
+    const int t = threadIdx.x;
+    if (blockIdx.x < RW) {
+        const int i = (blockIdx.x * 256 + t) * 4;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 14
+        for (int k = 0; k < slices; k++)
+            s += *reinterpret_cast<const f32x4 *>(wpart + (size_t)k * 3 * H * H + i);
+        const int l = i / (H * H);
+        const int o = (l == 0 ? OFF_W2 : l == 1 ? OFF_W3 : OFF_W4) + i % (H * H);
+#pragma unroll
+        for (int e = 0; e < 4; e++) grad[o + e] = s[e];
+        return;
+    }
+    __shared__ float red[8][32];
+    const int c = (blockIdx.x - RW) * 32 + (t & 31), rg = t >> 5;
     float s = 0.f;
-    const int64_t n = M * 4;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const float d = Y[i] - T[i];
-        dY[i] = 2.0f * d / (float)M;
-        s += d * d;
-    }
-    red[threadIdx.x] = s;
+    if (c < PT_N)
+#pragma unroll 8
+        for (int k = rg; k < tiles; k += 8) s += tpart[(size_t)k * PT_N + c];
+    red[rg][t & 31] = s;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// output layer backward: gW5[j][o] = sum_m H4[m][j] dY[m][o]; gb5[o] = sum_m dY[m][o];
-// dZ4[m][j] = (sum_o dY[m][o] W5[j][o]) silu'(Z4[m][j]).  One thread per (m, j)
-// for dZ4; the reductions over m run per column block with atomics.
-__global__ void k_out_backward_dz(const float *__restrict__ theta, const float *__restrict__ dY,
-                                  const __bf16 *__restrict__ Z4, int64_t M,
-                                  __bf16 *__restrict__ dZ4) {
-    const int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (idx >= M * H) return;
-    const int64_t m = idx / H;
-    const int j = (int)(idx % H);
-    float s = 0.f;
+    if (rg > 0 || c > PT_LOSS) return;
 #pragma unroll
-    for (int o = 0; o < 4; o++) s += dY[m * 4 + o] * theta[OFF_W5 + j * 4 + o];
-    dZ4[idx] = tobf(s * dsilu(frombf(Z4[idx])));
-}
-
-// column sums / small reductions: out[j*ncol_out + o] += sum_m X[m][j] Yv[m][o]
-// with X BF16 (M x nx, row stride nx) and Yv FP32 (M x ny).  Grid: (nx, chunks).
-__global__ void k_outer_reduce(const __bf16 *__restrict__ X, int nx, const float *__restrict__ Yv,
-                               int ny, int64_t M, float *__restrict__ out) {
-    const int j = blockIdx.x;
-    const int64_t chunk = (M + gridDim.y - 1) / gridDim.y;
-    const int64_t m_lo = blockIdx.y * chunk;
-    const int64_t m_hi = m_lo + chunk < M ? m_lo + chunk : M;
-    __shared__ float red[256][4];
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int64_t m = m_lo + threadIdx.x; m < m_hi; m += blockDim.x) {
-        const float xv = X ? frombf(X[m * nx + j]) : 1.0f;
-        for (int o = 0; o < ny; o++) s[o] += xv * Yv[m * ny + o];
-    }
-    for (int o = 0; o < 4; o++) red[threadIdx.x][o] = s[o];
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (threadIdx.x < st)
-            for (int o = 0; o < 4; o++) red[threadIdx.x][o] += red[threadIdx.x + st][o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int o = 0; o < ny; o++) atomicAdd(&out[j * ny + o], red[0][o]);
-}
-
-// Column reductions over the M rows of a BF16 (M x 256) matrix, one block per
-// CS_ROWS rows: thread t reads 8 adjacent columns (one 16-byte load) of rows
-// t / 32, t / 32 + 8, ...; the 8 row groups are summed in LDS and each block
-// adds its 256 partial sums with atomics.
-constexpr int CS_ROWS = 128;
-
-// bias gradients: gb[j] += sum_m dZ[m][j]
-__global__ __launch_bounds__(256) void k_colsum(const __bf16 *__restrict__ dZ, int64_t M,
-                                                float *__restrict__ gb) {
-    __shared__ float red[8][H];
-    const int t = threadIdx.x, c8 = 8 * (t & 31), rg = t >> 5;
-    const int64_t r0 = (int64_t)blockIdx.x * CS_ROWS;
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int r = rg; r < CS_ROWS; r += 8) {
-        const int64_t m = r0 + r;
-        if (m >= M) break;
-        const bf16x8 v = *reinterpret_cast<const bf16x8 *>(dZ + m * H + c8);
-#pragma unroll
-        for (int e = 0; e < 8; e++) s[e] += frombf(v[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; e++) red[rg][c8 + e] = s[e];
-    __syncthreads();
-    float tot = 0.f;
-#pragma unroll
-    for (int g = 0; g < 8; g++) tot += red[g][t];
-    atomicAdd(&gb[t], tot);
-}
-
-// Outer-product reduction of an (M x 4) FP32 and an (M x 256) BF16 matrix,
-// g[c][j] += sum_m feat[m][c] dZ1[m][j]: the first layer's weight gradient
-// (UNIT_MAJOR false, stored [4][256]) and the output layer's (feat = dY,
-// dZ1 = the last hidden activations, UNIT_MAJOR true, stored [256][4]).
-// Row-blocked like k_colsum: thread t reads 8 adjacent columns of every 8th
-// row with one 16-byte load.
-template <bool UNIT_MAJOR>
-__global__ __launch_bounds__(256) void k_outer4(const float *__restrict__ feat,
-                                                const __bf16 *__restrict__ dZ1, int64_t M,
-                                                float *__restrict__ gW1) {
-    __shared__ float red[8][4][H];
-    const int t = threadIdx.x, c8 = 8 * (t & 31), rg = t >> 5;
-    const int64_t r0 = (int64_t)blockIdx.x * CS_ROWS;
-    float s[4][8];
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) s[c][e] = 0.f;
-    for (int r = rg; r < CS_ROWS; r += 8) {
-        const int64_t m = r0 + r;
-        if (m >= M) break;
-        const bf16x8 v = *reinterpret_cast<const bf16x8 *>(dZ1 + m * H + c8);
-        const f32x4 f = *reinterpret_cast<const f32x4 *>(feat + m * 4);
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) s[c][e] += f[c] * frombf(v[e]);
-    }
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) red[rg][c][c8 + e] = s[c][e];
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        float tot = 0.f;
-#pragma unroll
-        for (int g = 0; g < 8; g++) tot += red[g][c][t];
-        atomicAdd(&gW1[UNIT_MAJOR ? t * 4 + c : c * H + t], tot);
-    }
+    for (int g = 1; g < 8; g++) s += red[g][t];
+    if (c < PT_B)
+        grad[OFF_W1 + c] = s;
+    else if (c < PT_W5) {
+        const int l = (c - PT_B) / H;
+        grad[(l == 0 ? OFF_B1 : l == 1 ? OFF_B2 : l == 2 ? OFF_B3 : OFF_B4) + (c - PT_B) % H] = s;
+    } else if (c < PT_B5)
+        grad[OFF_W5 + c - PT_W5] = s;
+    else if (c < PT_LOSS)
+        grad[OFF_B5 + c - PT_B5] = s;
+    else if (loss)
+        loss[0] = s;
 }
 
 // BF16 copies of W2..W4 (layout at BF_SW .. BF_TSWLO): fragment order of
-// the high parts, row-major high parts, fragment order of the low parts,
-// and fragment order of the transposes' high and low parts
+// the high and the low parts, and of the transposes' high and low parts
 __device__ __forceinline__ size_t frag_index(int k, int n) {
     // fragment order of V[k][n] (k input, n output): ((jt * 8 + ks) * 64 +
     // lane) * 8 + e with n = 16 jt + lane % 16, k = 32 ks + 8 (lane / 16) + e
@@ -953,35 +1027,40 @@ __device__ __forceinline__ size_t frag_index(int k, int n) {
     return (((size_t)jt * 8 + ks) * 64 + lane) * 8 + e;
 }
 
-__global__ void k_sync_bf16(const float *__restrict__ theta, __bf16 *__restrict__ wbf) {
-    const int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (idx >= 3 * H * H) return;
-    const int l = (int)(idx / (H * H));
-    const int rem = (int)(idx % (H * H));
+// the copies of parameter i, if it is a hidden weight
+__device__ __forceinline__ void sync_copies(int i, float v, __bf16 *__restrict__ wbf) {
+    const int l = i >= OFF_W4 ? 2 : i >= OFF_W3 ? 1 : 0;
+    const int rem = i - (l == 0 ? OFF_W2 : l == 1 ? OFF_W3 : OFF_W4);
+    if (rem < 0 || rem >= H * H) return;
     const int k = rem / H, n = rem % H;  // W[k][n], row-major [in][out]
-    const float v = theta[(l == 0 ? OFF_W2 : l == 1 ? OFF_W3 : OFF_W4) + rem];
     __bf16 hi, lo;
     split_bf(v, hi, lo);
     const size_t lb = (size_t)l * H * H;
     wbf[BF_SW + lb + frag_index(k, n)] = hi;
-    wbf[BF_ROW + lb + rem] = hi;
     wbf[BF_SWLO + lb + frag_index(k, n)] = lo;
     wbf[BF_TSW + lb + frag_index(n, k)] = hi;    // W^T[n][k] = W[k][n]
     wbf[BF_TSWLO + lb + frag_index(n, k)] = lo;
 }
 
-// Adam (FP32 masters)
-__global__ void k_adam(float *__restrict__ theta, const float *__restrict__ g,
-                       float *__restrict__ m, float *__restrict__ v, int64_t n, float lr,
-                       float b1, float b2, float eps, float c1, float c2) {
+__global__ void k_sync_bf16(const float *__restrict__ theta, __bf16 *__restrict__ wbf) {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    if (i < NPARAM) sync_copies((int)i, theta[i], wbf);
+}
+
+// Adam (FP32 masters), and the updated weights' BF16 copies
+__global__ void k_adam(float *__restrict__ theta, const float *__restrict__ g,
+                       float *__restrict__ m, float *__restrict__ v, float lr, float b1, float b2,
+                       float eps, float c1, float c2, __bf16 *__restrict__ wbf) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= NPARAM) return;
     const float gi = g[i];
     const float mi = b1 * m[i] + (1.0f - b1) * gi;
     const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    theta[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    const float th = theta[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    theta[i] = th;
+    sync_copies((int)i, th, wbf);
 }
 
 // training data: positions (3,M) FP64 with exact Phi and grad -> features
@@ -1152,24 +1231,11 @@ int check_norm(const gamd_mlp_norm *nm) {
 // twice as often (8,192 points: 35 against 27 us).  Same results either way.
 bool tile_points16(size_t M) { return M <= (size_t)cu_count() * 16; }
 
+// slices of the points in k_wgrad: whole stages, at most WG_SLICES
+int wgrad_slices(int64_t M) { return (int)(M / WG_P < WG_SLICES ? M / WG_P : WG_SLICES); }
+
 int check_params(const float *theta, const uint16_t *wbf) {
     return (theta && wbf) ? GAMD_OK : GAMD_ERR_INVALID;
-}
-
-// the training forward uses 66 KB of dynamic LDS (one padded 128 x 256 BF16
-// activation buffer), above the default 64 KB; raise its limit once per
-// process (a function-local static: initialised once even when several host
-// threads make their first call together)
-int ensure_lds() {
-    static const int rc = [] {
-        const void *ks[1] = {(const void *)k_mlp_forward_train};
-        for (const void *k : ks)
-            if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) !=
-                hipSuccess)
-                return (int)GAMD_ERR_HIP;
-        return (int)GAMD_OK;
-    }();
-    return rc;
 }
 
 }  // namespace
@@ -1180,15 +1246,15 @@ int64_t gamd_mlp_param_count(void) { return NPARAM; }
 int64_t gamd_mlp_bf16_count(void) { return NBF; }
 
 int64_t gamd_mlp_workspace_bytes(int64_t M) {
-    // Zs, Hs: 2 x 4 x M x 256 BF16; Y, dY: 2 x M x 4 FP32; dZ ping-pong 2 x M x 256 BF16;
-    // loss partials 1024 FP32
-    return 2 * 4 * M * H * 2 + 2 * M * 4 * 4 + 2 * M * H * 2 + 1024 * 4 + 256;
+    // H1..H3 and dZ2..dZ4 (6 x M x 256 BF16), the hidden gradients' partial
+    // matrices, one row of partial sums per tile
+    return 6 * M * H * 2 + (int64_t)wgrad_slices(M) * 3 * H * H * 4 + (M / TP) * PT_N * 4 + 256;
 }
 
 int gamd_mlp_sync_bf16(const float *theta, uint16_t *wbf, void *stream) {
     if (check_params(theta, wbf)) return GAMD_ERR_INVALID;
-    hipLaunchKernelGGL(k_sync_bf16, dim3(3 * H * H / 256), dim3(256), 0, as_stream(stream), theta,
-                       reinterpret_cast<__bf16 *>(wbf));
+    hipLaunchKernelGGL(k_sync_bf16, dim3(grid_for(NPARAM, 256)), dim3(256), 0, as_stream(stream),
+                       theta, reinterpret_cast<__bf16 *>(wbf));
     return launch_status();
 }
 
@@ -1223,57 +1289,18 @@ int gamd_mlp_gradients(const float *theta, const uint16_t *wbf, const float *fea
     if ((int64_t)workspace_bytes < gamd_mlp_workspace_bytes((int64_t)M)) return GAMD_ERR_INVALID;
     hipStream_t s = as_stream(stream);
     const int64_t Mi = (int64_t)M;
-    unsigned char *ws = static_cast<unsigned char *>(workspace);
-    __bf16 *Zs = reinterpret_cast<__bf16 *>(ws);
-    __bf16 *Hs = Zs + 4 * Mi * H;
-    float *Y = reinterpret_cast<float *>(Hs + 4 * Mi * H);
-    float *dY = Y + Mi * 4;
-    __bf16 *dZa = reinterpret_cast<__bf16 *>(dY + Mi * 4);
-    __bf16 *dZb = dZa + Mi * H;
-    float *partial = reinterpret_cast<float *>(dZb + Mi * H);
-    const __bf16 *wsw = reinterpret_cast<const __bf16 *>(wbf);
-    const __bf16 *wrow = wsw + 3 * H * H;
-    if (ensure_lds()) return GAMD_ERR_HIP;
-    GAMD_HIP_CHECK(hipMemsetAsync(grad, 0, NPARAM * sizeof(float), s));
-    hipLaunchKernelGGL(k_mlp_forward_train, dim3((unsigned)((Mi + TILE - 1) / TILE)), dim3(256),
-                       LDS_BYTES, s, theta, wsw, feat, Mi, Zs, Hs, Y);
-    const unsigned lblocks = 512;
-    hipLaunchKernelGGL(k_loss, dim3(lblocks), dim3(256), 0, s, Y, target, Mi, dY, partial);
-    // output layer
-    const unsigned cs_blocks = (unsigned)((Mi + CS_ROWS - 1) / CS_ROWS);
-    hipLaunchKernelGGL(k_outer4<true>, dim3(cs_blocks), dim3(256), 0, s, dY, Hs + 3 * Mi * H, Mi,
-                       grad + OFF_W5);
-    hipLaunchKernelGGL(k_outer_reduce, dim3(1, 16), dim3(256), 0, s, (const __bf16 *)nullptr, 1, dY,
-                       4, Mi, grad + OFF_B5);
-    hipLaunchKernelGGL(k_out_backward_dz, dim3(grid_for(Mi * H, 256)), dim3(256), 0, s, theta, dY,
-                       Zs + 3 * Mi * H, Mi, dZa);
-    // hidden layers 4, 3, 2: dW_l = H_{l-1}^T dZ_l, db_l, dZ_{l-1} = (dZ_l W_l^T) silu'(Z_{l-1})
-    __bf16 *dZ = dZa, *dZn = dZb;
-    const int offW[3] = {OFF_W2, OFF_W3, OFF_W4}, offB[3] = {OFF_B2, OFF_B3, OFF_B4};
-    for (int l = 2; l >= 0; l--) {  // l indexes W_{l+2}
-        const __bf16 *Hin = Hs + (size_t)l * Mi * H;   // H_{l+1}
-        // split the points over up to 16 slices of whole 64-point stages (grad is zeroed above)
-        unsigned ksplit = 16;
-        while (ksplit > 1 && Mi % (WG_KC * (int64_t)ksplit) != 0) ksplit /= 2;
-        hipLaunchKernelGGL(k_wgrad, dim3(H / 64, H / 64, ksplit), dim3(256), 0, s, (int)Mi, Hin, dZ,
-                           grad + offW[l], grad + offB[l]);
-        hipLaunchKernelGGL((k_gemm<1, true>), dim3((unsigned)(Mi / 64), H / 64), dim3(256), 0, s, (int)Mi, H,
-                           H, dZ, (int64_t)H, (int64_t)1, wrow + (size_t)l * H * H, (int64_t)1,
-                           (int64_t)H, (float *)nullptr, dZn, (int64_t)H, Zs + (size_t)l * Mi * H);
-        __bf16 *tmp = dZ;
-        dZ = dZn;
-        dZn = tmp;
-    }
-    // first layer
-    hipLaunchKernelGGL(k_outer4<false>, dim3(cs_blocks), dim3(256), 0, s, feat, dZ, Mi,
-                       grad + OFF_W1);
-    hipLaunchKernelGGL(k_colsum, dim3(cs_blocks), dim3(256), 0, s, dZ, Mi, grad + OFF_B1);
-    if (loss) {
-        // sum of the per-block partials into loss[0]
-        GAMD_HIP_CHECK(hipMemsetAsync(loss, 0, sizeof(float), s));
-        hipLaunchKernelGGL(k_outer_reduce, dim3(1, 1), dim3(256), 0, s, (const __bf16 *)nullptr, 1,
-                           partial, 1, (int64_t)lblocks, loss);
-    }
+    const int slices = wgrad_slices(Mi), tiles = (int)(Mi / TP);
+    __bf16 *Hs = static_cast<__bf16 *>(workspace);
+    __bf16 *Ds = Hs + 3 * Mi * H;
+    float *wpart = reinterpret_cast<float *>(Ds + 3 * Mi * H);
+    float *tpart = wpart + (size_t)slices * 3 * H * H;
+    const __bf16 *w = reinterpret_cast<const __bf16 *>(wbf);
+    hipLaunchKernelGGL(k_train_tile, dim3((unsigned)tiles), dim3(256), 0, s, theta, w, feat,
+                       target, Mi, Hs, Ds, tpart);
+    hipLaunchKernelGGL(k_wgrad, dim3(16 * grid_for(3 * slices, 8)), dim3(512), 0, s, Mi, slices,
+                       Hs, Ds, wpart);
+    hipLaunchKernelGGL(k_grad_reduce, dim3(RW + RP), dim3(256), 0, s, wpart, slices, tpart, tiles,
+                       grad, loss);
     return launch_status();
 }
 
@@ -1283,10 +1310,8 @@ int gamd_mlp_adam(float *theta, const float *grad, float *m, float *v, int64_t s
     const float c1 = 1.0f / (1.0f - powf(beta1, (float)step));
     const float c2 = 1.0f / (1.0f - powf(beta2, (float)step));
     hipLaunchKernelGGL(k_adam, dim3(grid_for(NPARAM, 256)), dim3(256), 0, as_stream(stream), theta,
-                       grad, m, v, (int64_t)NPARAM, lr, beta1, beta2, eps, c1, c2);
-    int rc = launch_status();
-    if (rc) return rc;
-    return gamd_mlp_sync_bf16(theta, wbf, stream);
+                       grad, m, v, lr, beta1, beta2, eps, c1, c2, reinterpret_cast<__bf16 *>(wbf));
+    return launch_status();
 }
 
 int gamd_surrogate_leapfrog_step(const float *theta, const uint16_t *wbf, const gamd_mlp_norm *norm,

@@ -386,7 +386,7 @@ int64_t gamd_mlp_bf16_count(void);
 /* bytes of workspace gamd_mlp_gradients needs for a batch of M points */
 int64_t gamd_mlp_workspace_bytes(int64_t M);
 /* BF16 copies of the hidden weights (high and low parts in matrix-core
- * fragment order, their transposes, and row-major high parts) */
+ * fragment order, and their transposes) */
 int gamd_mlp_sync_bf16(const float *theta, uint16_t *wbf, void *stream);
 /* inference: q (3,M) FP64 -> Phi_net (M) and grad Phi_net (3,M) FP64, the
  * hidden products carried to ~16 significant bits (three BF16 products of

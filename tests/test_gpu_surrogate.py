@@ -131,6 +131,45 @@ def test_gradients_match_oracle():
         assert rel < 6e-2, (name, rel)
 
 
+@pytest.mark.parametrize("M", [64, 128, 2688, 2752, 4096, 5440])
+def test_gradients_count_every_tile_once(M):
+    """One 64-point tile, a few, as many stages as the weight gradients have
+    slices, one more, and uneven slices.  Every point's error signals depend
+    on that point alone, so the batch in reverse order (each point in another
+    lane, tile and slice) gives the same gradient and loss up to the order of
+    FP32 sums of M terms, M 2^-24.  Where M / 64 is a power of two a tile taken
+    alone has the same signals but for that factor, and the batch equals the
+    sum over its tiles to the same bound.  A lost or doubled tile is off by
+    1 / 85 at least."""
+    from gala_amd import _device as dev
+    t = dev.torch()
+    sur, pot, S, T = _surrogate(4)
+    rng = np.random.default_rng(M)
+    feat = dev.to_dev(rng.normal(size=(M, 4)), dtype=t.float32)
+    target = dev.to_dev(rng.normal(size=(M, 4)), dtype=t.float32)
+
+    def run(f, y):
+        loss, g = sur.gradients(f.contiguous(), y.contiguous())
+        return float(loss.item()), dev.to_host(g).astype(np.float64)
+
+    def close(a, b):
+        assert abs(a[0] - b[0]) <= M * 2.0 ** -24 * b[0]
+        for (name, _), i, j in zip(OM.SHAPES, offsets[:-1], offsets[1:]):
+            rel = np.linalg.norm(a[1][i:j] - b[1][i:j]) / np.linalg.norm(b[1][i:j])
+            assert rel <= M * 2.0 ** -24, (name, rel)
+
+    offsets = np.cumsum([0] + [int(np.prod(s)) for _, s in OM.SHAPES])
+    whole = run(feat, target)
+    again = run(feat, target)
+    assert again[0] == whole[0]  # the order of the sums is fixed
+    np.testing.assert_array_equal(again[1], whole[1])
+    close(run(feat.flip(0), target.flip(0)), whole)
+    tiles = M // 64
+    if tiles & (tiles - 1) == 0:
+        parts = [run(feat[i:i + 64], target[i:i + 64]) for i in range(0, M, 64)]
+        close((sum(p[0] for p in parts), sum(p[1] for p in parts) / tiles), whole)
+
+
 def test_training_beats_monopole_and_falls_back():
     """A short training run: the loss falls, the trained network's force
     -grad Phi_net beats the monopole-only approximation (the method without
