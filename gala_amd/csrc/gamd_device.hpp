@@ -14,6 +14,7 @@
 #include <stdint.h>
 
 #include "gala_amd.h"
+#include "gamd_scf.hpp"
 
 namespace gamd {
 
@@ -27,7 +28,7 @@ struct DevComp {
     double d[4];          // host-folded constants, see fold_component()
     double q0[3];
     double R[9];
-    const double *coef;   // SCF: device, per (l, m) block: (S_nlm, T_nlm) for n = 0..nmax
+    const double *coef;   // SCF: device, the table of gamd_scf.hpp
 };
 
 struct DevPot {
@@ -43,9 +44,10 @@ struct DevPot {
 // dependent sqrt/divide/log chains run one after the other; written out
 // straight, the scheduler interleaves them, which is what a lone lane in the
 // tail of a persistent launch needs.
-// MW: Hernquist, Hernquist, MN, NFW, unshifted.  SCF106: one unshifted SCF
-// component with nmax = 10, lmax = 6 (the expansion inlined and unrolled).
-enum { LAYOUT_GENERIC = 0, LAYOUT_MW = 1, LAYOUT_SCF106 = 2 };
+// MW: Hernquist, Hernquist, MN, NFW, unshifted.  SCF: one unshifted SCF
+// component of any size; SCF106: the same with nmax = 10, lmax = 6, written out
+// whole.
+enum { LAYOUT_GENERIC = 0, LAYOUT_MW = 1, LAYOUT_SCF106 = 2, LAYOUT_SCF = 3 };
 
 // ---------------------------------------------------------------------------
 // Natural log with a short dependency chain, for finite x > 0.  The library
@@ -284,257 +286,56 @@ __device__ __forceinline__ void comp_hessian_analytic(const DevComp &c, double x
 }
 
 // ---------------------------------------------------------------------------
-// SCF basis expansion (Hernquist-Ostriker, Lowing+2011 real coefficients):
-// the quantity gala computes term by term in bfe.cpp:114-189 with GSL calls
-// per (n,l,m) (bfe_helper.cpp:24-90), reorganised for a GPU lane:
-//   * cos(m phi), sin(m phi) by the angle-addition recurrence from x/R, y/R;
-//   * normalised Y_lm(cos theta) and dY_lm/dtheta by the standard stable
-//     recurrences (one pass over l, m);
-//   * per l, Gegenbauer C_n^{(2l+3/2)}(xi) and C_{n-1}^{(2l+5/2)}(xi) by their
-//     three-term recurrences, giving phi_nl(s) and dphi_nl/ds for all n;
-//   * the n-sums A_lm = sum_n phi_nl S_nlm (and T, and the s-derivatives)
-//     are FMA chains over coefficients read with wave-uniform (scalar) loads.
-// coef layout: for l = 0..lmax, m = 0..l, n = 0..nmax: (S_nlm, T_nlm).
-// Returns Phi / (G M / r_s) scaled; accumulates G M/r_s^2 * grad into g.
-
-// 1/n for the Gegenbauer recurrences (n <= GAMD_SCF_MAX_NMAX + 1): a
-// wave-uniform table read instead of two FP64 divisions per (l, n) term
-static __constant__ double scf_inv_n[GAMD_SCF_MAX_NMAX + 2] = {0.0, 1.0 / 1.0, 1.0 / 2.0, 1.0 / 3.0, 1.0 / 4.0, 1.0 / 5.0, 1.0 / 6.0, 1.0 / 7.0, 1.0 / 8.0, 1.0 / 9.0, 1.0 / 10.0, 1.0 / 11.0, 1.0 / 12.0, 1.0 / 13.0, 1.0 / 14.0, 1.0 / 15.0, 1.0 / 16.0, 1.0 / 17.0, 1.0 / 18.0, 1.0 / 19.0, 1.0 / 20.0, 1.0 / 21.0};
-
-// Position of (S_nlm, T_nlm) in the device coefficient table: per l, per n,
-// the l + 1 pairs of m = 0..l contiguous, so one n step of the expansion reads
-// one contiguous run of 2 (l + 1) doubles (wide scalar loads).
-__host__ __device__ __forceinline__ int scf_pack_index(int l, int m, int n, int nmax) {
-    return (nmax + 1) * (l * (l + 1) / 2) + n * (l + 1) + m;
+// SCF basis expansion (gamd_scf.hpp): one out-of-line copy per kernel of the
+// value and of the gradient.  The sum is long, and inlining it at each of
+// DOP853's stage evaluations would multiply code size (and compile time) with
+// no gain, since the call overhead is small next to the sum.
+// The table and sizes are those of one component of a potential, the same in
+// every lane that calls; arguments arrive in vector registers and return to
+// scalar ones here.
+__device__ __forceinline__ const double *wave_uniform(const double *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return reinterpret_cast<const double *>(((uint64_t)hi << 32) | lo);
 }
 
-// The Gegenbauer recurrence factors of scf_eval_t as a table over (l, n):
-// for a = 2l + 3/2 and b = a + 1, [0] = n + a - 1, [1] = n + 2a - 2,
-// [2] = n + b - 1, [3] = n + 2b - 2 (the same doubles the loop would form from
-// its counter), so the loop reads them instead of converting and adding.
-struct ScfRecTable {
-    double f[GAMD_SCF_MAX_LMAX + 1][GAMD_SCF_MAX_NMAX + 2][4];
-};
-constexpr ScfRecTable scf_rec_table() {
-    ScfRecTable t{};
-    for (int l = 0; l <= GAMD_SCF_MAX_LMAX; l++) {
-        const double a = 2.0 * l + 1.5, b = a + 1.0;
-        for (int n = 0; n <= GAMD_SCF_MAX_NMAX + 1; n++) {
-            t.f[l][n][0] = n + a - 1.0;
-            t.f[l][n][1] = n + 2.0 * a - 2.0;
-            t.f[l][n][2] = n + b - 1.0;
-            t.f[l][n][3] = n + 2.0 * b - 2.0;
-        }
-    }
-    return t;
-}
-static __constant__ ScfRecTable scf_rec = scf_rec_table();
-
-template <int NMAX, int LMAX>
-__device__ __forceinline__ void scf_eval_t(const double *__restrict__ cf, double G, double M,
-                                           double rs, int nmax_rt, int lmax_rt, double x,
-                                           double y, double z, bool want_grad, double &phi_out,
-                                           double &gx, double &gy, double &gz) {
-    const int nmax = NMAX >= 0 ? NMAX : nmax_rt;
-    const int lmax = LMAX >= 0 ? LMAX : lmax_rt;
-    // the coefficients are read-only for the whole launch and every lane reads
-    // the same one: through the constant address space they become scalar
-    // (SMEM) loads instead of a vector load and wait per term
-    const __attribute__((address_space(4))) double *cfc =
-        (const __attribute__((address_space(4))) double *)cf;
-    const double FOURPI_SQRT = 3.544907701811031;
-    const double R2 = x * x + y * y;
-    const double r2 = R2 + z * z;
-    const double r = sqrt(r2);
-    const double Rc = sqrt(R2);
-    const double s = r / rs;
-    const double X = z / r;          // cos(theta)
-    const double sinth = Rc / r;     // sin(theta)
-    double cphi = 1.0, sphi = 0.0;   // atan2(0, 0) = 0 on the axis, as gala
-    if (Rc > 0.0) {
-        cphi = x / Rc;
-        sphi = y / Rc;
-    }
-    const double ops = 1.0 + s;
-    const double inv_ops = 1.0 / ops;
-    const double inv_s = 1.0 / s;
-    const double xi = (s - 1.0) * inv_ops;
-    const double inv_ops2 = inv_ops * inv_ops;
-
-    double Phi = 0.0, dr = 0.0, dth = 0.0, dph = 0.0;
-
-    // running radial prefactor pre_l = -sqrt(4 pi) s^l (1+s)^(-2l-1)
-    double pre = -FOURPI_SQRT / ops;
-    // normalised Y_mm seeds: Y_00 = 1/sqrt(4 pi)
-    double ymm = 1.0 / FOURPI_SQRT;
-    // cos(m phi), sin(m phi) for m = 0..lmax kept in registers
-    double cm[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-    double sm[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-    cm[0] = 1.0;
-    sm[0] = 0.0;
-#pragma unroll
-    for (int m = 1; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-        if (m <= lmax) {
-            cm[m] = cm[m - 1] * cphi - sm[m - 1] * sphi;
-            sm[m] = sm[m - 1] * cphi + cm[m - 1] * sphi;
-        }
-    }
-    // Y_{l-1,m} and Y_{l-2,m} for every m, updated as l advances
-    double y1[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-    double y2[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-#pragma unroll
-    for (int m = 0; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-        y1[m] = 0.0;
-        y2[m] = 0.0;
-    }
-
-#pragma unroll
-    for (int l = 0; l <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); l++) {
-        if (l > lmax) break;
-        // radial functions for this l: phi_nl = pre * C_n^{a}(xi), a = 2l + 3/2
-        // dphi_nl/ds = pre * [ (l/s - (2l+1)/(1+s)) C_n^{a} + 2a C_{n-1}^{a+1} 2/(1+s)^2 ]
-        const double a = 2.0 * l + 1.5;
-        const double dlog = (l == 0 ? 0.0 : l * inv_s) - (2.0 * l + 1.0) * inv_ops;
-        const double chain = 4.0 * a * inv_ops2;
-        // Y_lm for all m <= l at this l
-        double ylm[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-        // n-sums per m
-        double As[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-        double Bs[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-        double dAs[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-        double dBs[LMAX >= 0 ? LMAX + 1 : GAMD_SCF_MAX_LMAX + 1];
-#pragma unroll
-        for (int m = 0; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-            As[m] = 0.0;
-            Bs[m] = 0.0;
-            dAs[m] = 0.0;
-            dBs[m] = 0.0;
-        }
-        // Gegenbauer recurrences in n
-        double c0 = 1.0, c1 = 0.0;  // C_n^a, C_{n-1}^a
-        double e0 = 0.0, e1 = 0.0;  // C_{n-1}^{a+1}, C_{n-2}^{a+1}
-        // the fixed-size evaluator unrolls n by 10 (measured best for nmax 10;
-        // fully unrolled, the loop spills); the runtime-size one keeps a loop
-#pragma unroll(NMAX >= 0 ? 10 : 1)
-        for (int n = 0; n <= nmax; n++) {
-            double Cn, En;  // C_n^a(xi), C_{n-1}^{a+1}(xi)
-            if (n == 0) {
-                Cn = 1.0;
-                En = 0.0;
-            } else if (n == 1) {
-                Cn = 2.0 * a * xi;
-                En = 1.0;
-            } else {
-                const double *rn = scf_rec.f[l][n], *rk = scf_rec.f[l][n - 1];
-                Cn = (2.0 * xi * rn[0] * c0 - rn[1] * c1) * scf_inv_n[n];
-                const double b = a + 1.0;
-                const int k = n - 1;  // index of E
-                En = (k == 1) ? 2.0 * b * xi
-                              : (2.0 * xi * rk[2] * e0 - rk[3] * e1) * scf_inv_n[k];
-            }
-            c1 = c0;
-            c0 = Cn;
-            e1 = e0;
-            e0 = En;
-            const double phinl = pre * Cn;
-            const double dphinl = pre * (dlog * Cn + chain * En);
-#pragma unroll
-            for (int m = 0; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-                if (m <= l) {
-                    const double S = cfc[2 * scf_pack_index(l, m, n, nmax)];
-                    const double T = cfc[2 * scf_pack_index(l, m, n, nmax) + 1];
-                    As[m] = fma(phinl, S, As[m]);
-                    Bs[m] = fma(phinl, T, Bs[m]);
-                    dAs[m] = fma(dphinl, S, dAs[m]);
-                    dBs[m] = fma(dphinl, T, dBs[m]);
-                }
-            }
-        }
-        // Y_lm(X) for this l (normalised, Condon-Shortley phase)
-#pragma unroll
-        for (int m = 0; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-            if (m <= l) {
-                double v;
-                if (m == l) {
-                    v = ymm;
-                } else if (m == l - 1) {
-                    v = sqrt(2.0 * m + 3.0) * X * y1[m];
-                } else {
-                    const double l2 = (double)l * l, m2 = (double)m * m;
-                    const double al = sqrt((4.0 * l2 - 1.0) / (l2 - m2));
-                    const double bl = sqrt(((l - 1.0) * (l - 1.0) - m2) / (4.0 * (l - 1.0) * (l - 1.0) - 1.0));
-                    v = al * (X * y1[m] - bl * y2[m]);
-                }
-                ylm[m] = v;
-            }
-        }
-        // accumulate
-#pragma unroll
-        for (int m = 0; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-            if (m <= l) {
-                const double ac = As[m] * cm[m] + Bs[m] * sm[m];
-                Phi = fma(ylm[m], ac, Phi);
-                if (want_grad) {
-                    const double dac = dAs[m] * cm[m] + dBs[m] * sm[m];
-                    dr = fma(ylm[m], dac, dr);
-                    // dY_lm/dtheta * sin(theta) = l X Y_lm - sqrt((2l+1)/(2l-1) (l-m)(l+m)) Y_{l-1,m}
-                    double dy = l * X * ylm[m];
-                    if (m < l)
-                        dy -= sqrt((2.0 * l + 1.0) / (2.0 * l - 1.0) * (double)(l - m) * (l + m)) * y1[m];
-                    dth = fma(dy, ac, dth);
-                    dph = fma((double)m * ylm[m], Bs[m] * cm[m] - As[m] * sm[m], dph);
-                }
-            }
-        }
-        // shift Y history, next Y_mm seed, next radial prefactor
-#pragma unroll
-        for (int m = 0; m <= (LMAX >= 0 ? LMAX : GAMD_SCF_MAX_LMAX); m++) {
-            if (m <= l) {
-                y2[m] = y1[m];
-                y1[m] = ylm[m];
-            }
-        }
-        ymm = -sqrt((2.0 * l + 3.0) / (2.0 * l + 2.0)) * sinth * ymm;
-        pre = pre * s * inv_ops2;
-    }
-    const double GMr = G * M / rs;
-    phi_out = Phi * GMr;
-    if (want_grad) {
-        // (d/dr, (1/r) d/dtheta, 1/(r sin theta) d/dphi) in units of r_s, then Cartesian
-        const double g_r = dr;
-        const double g_t = dth / (s * sinth);
-        const double g_p = dph / (s * sinth);
-        const double fac = G * M / (rs * rs);
-        gx += (sinth * cphi * g_r + X * cphi * g_t - sphi * g_p) * fac;
-        gy += (sinth * sphi * g_r + X * sphi * g_t + cphi * g_p) * fac;
-        gz += (X * g_r - sinth * g_t) * fac;
-    }
-}
-
-// One out-of-line copy per kernel: the SCF sum is long, and inlining it at
-// each of DOP853's stage evaluations would multiply code size (and compile
-// time) with no gain, since the call overhead is small next to the sum.
-// Returns (Phi, dPhi/dx, dPhi/dy, dPhi/dz).
-__device__ __noinline__ double4 scf_call(const double *__restrict__ cf, double G, double M,
+__device__ __noinline__ double scf_value(const double *__restrict__ table, double G, double M,
                                          double rs, int nmax, int lmax, double x, double y,
-                                         double z, int want_grad) {
-    double phi = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
+                                         double z) {
+    table = wave_uniform(table);
+    nmax = __builtin_amdgcn_readfirstlane(nmax);
+    lmax = __builtin_amdgcn_readfirstlane(lmax);
+    double phi, gx, gy, gz;
     if (nmax == 10 && lmax == 6)
-        scf_eval_t<10, 6>(cf, G, M, rs, 10, 6, x, y, z, want_grad != 0, phi, gx, gy, gz);
+        scf_field<10, 6, true, false>(table, G, M, rs, 10, 6, x, y, z, phi, gx, gy, gz);
     else
-        scf_eval_t<-1, -1>(cf, G, M, rs, nmax, lmax, x, y, z, want_grad != 0, phi, gx, gy, gz);
-    return make_double4(phi, gx, gy, gz);
+        scf_field<-1, GAMD_SCF_MAX_LMAX, true, false>(table, G, M, rs, nmax, lmax, x, y, z, phi,
+                                                      gx, gy, gz);
+    return phi;
 }
 
-__device__ __forceinline__ void scf_eval(const DevComp &c, double x, double y, double z,
-                                         bool want_grad, double &phi, double &gx, double &gy,
-                                         double &gz) {
-    const double4 r = scf_call(c.coef, c.p[0], c.p[1], c.p[2], c.nmax, c.lmax, x, y, z,
-                               want_grad ? 1 : 0);
-    phi = r.x;
-    gx += r.y;
-    gy += r.z;
-    gz += r.w;
+__device__ __noinline__ double3 scf_grad(const double *__restrict__ table, double G, double M,
+                                         double rs, int nmax, int lmax, double x, double y,
+                                         double z) {
+    table = wave_uniform(table);
+    nmax = __builtin_amdgcn_readfirstlane(nmax);
+    lmax = __builtin_amdgcn_readfirstlane(lmax);
+    double phi, gx, gy, gz;
+    if (nmax == 10 && lmax == 6)
+        scf_field<10, 6, false, true>(table, G, M, rs, 10, 6, x, y, z, phi, gx, gy, gz);
+    else
+        scf_field<-1, GAMD_SCF_MAX_LMAX, false, true>(table, G, M, rs, nmax, lmax, x, y, z, phi,
+                                                      gx, gy, gz);
+    return make_double3(gx, gy, gz);
+}
+
+__device__ __forceinline__ void scf_add_grad(const DevComp &c, double x, double y, double z,
+                                             double &gx, double &gy, double &gz) {
+    const double3 g = scf_grad(c.coef, c.p[0], c.p[1], c.p[2], c.nmax, c.lmax, x, y, z);
+    gx += g.x;
+    gy += g.y;
+    gz += g.z;
 }
 
 // SCF density (bfe.cpp:20-59): rho_nl = K_nl/(2 pi) sqrt(4 pi) s^l / (s (1+s)^(2l+3)) C_n(xi)
@@ -560,6 +361,7 @@ __device__ inline double scf_density(const DevComp &c, double x, double y, doubl
     }
     for (int m = 0; m <= lmax; m++) y1[m] = y2[m] = 0.0;
     double ymm = 1.0 / FOURPI_SQRT, rho = 0.0;
+    const double *table = c.coef;  // the block of l
     double pre = FOURPI_SQRT / (2.0 * PI) / (s * ops * ops * ops);  // s^l/(s (1+s)^(2l+3)) at l=0
     for (int l = 0; l <= lmax; l++) {
         const double a = 2.0 * l + 1.5;
@@ -579,9 +381,9 @@ __device__ inline double scf_density(const DevComp &c, double x, double y, doubl
                 c0 = Cn;
                 const double Knl = 0.5 * n * (n + 4 * l + 3) + (l + 1) * (2 * l + 1);
                 const double rnl = Knl * pre * Cn;
-                const int idx = 2 * scf_pack_index(l, m, n, nmax);
-                A += rnl * c.coef[idx];
-                B += rnl * c.coef[idx + 1];
+                const double *st = table + n * scf_row(l) + SCF_ROW_HEAD;
+                A += rnl * st[m == 0 ? 0 : 2 * m - 1];
+                B += rnl * (m == 0 ? 0.0 : st[2 * m]);  // sin(0 phi) = 0
             }
             rho += v * (A * cm[m] + B * sm[m]);
             y2[m] = y1[m];
@@ -589,6 +391,7 @@ __device__ inline double scf_density(const DevComp &c, double x, double y, doubl
         }
         ymm = -sqrt((2.0 * l + 3.0) / (2.0 * l + 2.0)) * sinth * ymm;
         pre = pre * s / (ops * ops);
+        table += (nmax + 1) * scf_row(l) + 1 + 3 * l;
     }
     return rho * M / (rs * rs * rs);
 }
@@ -615,10 +418,7 @@ __device__ __forceinline__ void comp_grad(const DevComp &c, double x, double y, 
         nfw_grad(c, x, y, z, sqrt(x * x + y * y + z * z), gx, gy, gz);
         break;
     case GAMD_SCF:
-        if (WITH_SCF) {
-            double phi;
-            scf_eval(c, x, y, z, true, phi, gx, gy, gz);
-        }
+        if (WITH_SCF) scf_add_grad(c, x, y, z, gx, gy, gz);
         break;
     default:
         break;
@@ -652,10 +452,7 @@ __device__ __forceinline__ void pot_grad(const DevPot &P, double x, double y, do
             case GAMD_MIYAMOTONAGAI: mn_grad(c, x, y, z, gx, gy, gz); break;
             case GAMD_NFW: nfw_grad(c, x, y, z, r, gx, gy, gz); break;
             case GAMD_SCF:
-                if (WITH_SCF) {
-                    double phi;
-                    scf_eval(c, x, y, z, true, phi, gx, gy, gz);
-                }
+                if (WITH_SCF) scf_add_grad(c, x, y, z, gx, gy, gz);
                 break;
             default: break;
             }
@@ -794,22 +591,28 @@ __device__ __forceinline__ void pot_grad_l(const DevPot &P, double x, double y, 
     } else if (LAYOUT == LAYOUT_SCF106) {
         const DevComp &c = P.c[0];
         double phi;
-        gx = 0.0;
-        gy = 0.0;
-        gz = 0.0;
-        scf_eval_t<10, 6>(c.coef, c.p[0], c.p[1], c.p[2], 10, 6, x, y, z, true, phi, gx, gy, gz);
+        scf_field<10, 6, false, true>(c.coef, c.p[0], c.p[1], c.p[2], 10, 6, x, y, z, phi, gx, gy,
+                                      gz);
+    } else if (LAYOUT == LAYOUT_SCF) {
+        const DevComp &c = P.c[0];
+        double phi;
+        scf_field<-1, GAMD_SCF_MAX_LMAX, false, true>(c.coef, c.p[0], c.p[1], c.p[2], c.nmax,
+                                                      c.lmax, x, y, z, phi, gx, gy, gz);
     } else {
         pot_grad<WITH_SCF>(P, x, y, z, gx, gy, gz);
     }
 }
 
+// waves per SIMD that the registers of an inlined expansion leave room for
+// (168 VGPRs written out whole, which is three; 228 with any size)
+constexpr int scf_waves(int layout) {
+    return layout == LAYOUT_SCF106 || layout == LAYOUT_SCF ? 2 : 1;
+}
+
 template <bool WITH_SCF>
 __device__ __forceinline__ double comp_value(const DevComp &c, double x, double y, double z) {
-    if (WITH_SCF && c.type == GAMD_SCF) {
-        double phi, gx = 0, gy = 0, gz = 0;
-        scf_eval(c, x, y, z, false, phi, gx, gy, gz);
-        return phi;
-    }
+    if (WITH_SCF && c.type == GAMD_SCF)
+        return scf_value(c.coef, c.p[0], c.p[1], c.p[2], c.nmax, c.lmax, x, y, z);
     return comp_value_analytic(c, x, y, z);
 }
 

@@ -22,6 +22,8 @@
 // 0 * NaN turns the velocity into NaN).
 #include <math.h>
 
+#include <type_traits>
+
 #include "gamd_host.hpp"
 
 using namespace gamd;
@@ -31,7 +33,7 @@ namespace {
 // RESUME: w0 holds positions and HALF-STEP velocities (the state the loop
 // carries between steps), so the initial half kick is skipped
 template <bool SCF, bool SAVE, int LAY, bool RESUME = false>
-__global__ __launch_bounds__(256) void k_leapfrog(const DevPot *__restrict__ Pp, const double *__restrict__ w0,
+__global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_leapfrog(const DevPot *__restrict__ Pp, const double *__restrict__ w0,
                                                   int64_t N, double dt, int64_t n_steps,
                                                   const int64_t *__restrict__ nsteps_i,
                                                   int64_t stride, int64_t nsave,
@@ -99,7 +101,7 @@ struct Ruth4Coef {
 };
 
 template <bool SCF, bool SAVE, int LAY>
-__global__ __launch_bounds__(256) void k_ruth4(const DevPot *__restrict__ Pp, const double *__restrict__ w0,
+__global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_ruth4(const DevPot *__restrict__ Pp, const double *__restrict__ w0,
                                                int64_t N, double dt, int64_t n_steps, int64_t stride,
                                                int64_t nsave, Ruth4Coef cf, double *__restrict__ wout,
                                                double *__restrict__ wfinal) {
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(256) void k_ruth4(const DevPot *__restrict__ Pp, co
         x = x + cf.c[0] * vx * dt;
         y = y + cf.c[0] * vy * dt;
         z = z + cf.c[0] * vz * dt;
-#pragma unroll
+#pragma unroll(SCF ? 1 : 3)
         for (int k = 1; k < 4; k++) {
             double gx, gy, gz;
             pot_grad_l<SCF, LAY>(P, x, y, z, gx, gy, gz);
@@ -156,6 +158,22 @@ __global__ __launch_bounds__(256) void k_ruth4(const DevPot *__restrict__ Pp, co
     }
 }
 
+// f(has_scf, layout) with both as compile-time constants, for the kernels of a
+// potential's layout
+template <class F>
+auto by_layout(const gamd_potential *pot, F f) {
+    using T = std::true_type;
+    using N = std::false_type;
+    switch (pot->dev.layout) {
+    case LAYOUT_MW: return f(N{}, std::integral_constant<int, LAYOUT_MW>{});
+    case LAYOUT_SCF106: return f(T{}, std::integral_constant<int, LAYOUT_SCF106>{});
+    case LAYOUT_SCF: return f(T{}, std::integral_constant<int, LAYOUT_SCF>{});
+    default:
+        return pot->dev.has_scf ? f(T{}, std::integral_constant<int, LAYOUT_GENERIC>{})
+                                : f(N{}, std::integral_constant<int, LAYOUT_GENERIC>{});
+    }
+}
+
 constexpr unsigned LF_BLOCK = 64;  // one wave per workgroup spreads small N over all CUs
 
 // ---------------------------------------------------------------------------
@@ -178,7 +196,7 @@ struct ChunkArgs {
 };
 
 template <bool SCF, int LAY>
-__global__ __launch_bounds__(256) void k_leapfrog_chunk(const DevPot *__restrict__ Pp, ChunkArgs a) {
+__global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_leapfrog_chunk(const DevPot *__restrict__ Pp, ChunkArgs a) {
     const DevPot &P = *Pp;
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= a.N) return;
@@ -319,17 +337,9 @@ extern "C" int gamd_leapfrog(const gamd_potential *pot, const double *w0, size_t
     const int64_t nsave = w_out ? n_steps / save_stride + 1 : 0;
     const unsigned g = grid_for(N, LF_BLOCK);
     hipStream_t s = as_stream(stream);
-    const bool scf = pot->dev.has_scf;
-    const bool mw = pot->dev.layout == LAYOUT_MW;
-    const bool scf106 = pot->dev.layout == LAYOUT_SCF106;
-    auto kern = w_out ? (scf106 ? k_leapfrog<true, true, LAYOUT_SCF106>
-                         : scf  ? k_leapfrog<true, true, LAYOUT_GENERIC>
-                         : mw   ? k_leapfrog<false, true, LAYOUT_MW>
-                                : k_leapfrog<false, true, LAYOUT_GENERIC>)
-                      : (scf106 ? k_leapfrog<true, false, LAYOUT_SCF106>
-                         : scf  ? k_leapfrog<true, false, LAYOUT_GENERIC>
-                         : mw   ? k_leapfrog<false, false, LAYOUT_MW>
-                                : k_leapfrog<false, false, LAYOUT_GENERIC>);
+    auto kern = by_layout(pot, [&](auto scf, auto lay) {
+        return w_out ? k_leapfrog<scf.value, true, lay.value> : k_leapfrog<scf.value, false, lay.value>;
+    });
     hipLaunchKernelGGL(kern, dim3(g), dim3(LF_BLOCK), 0, s, pot->ddev, w0, (int64_t)N, dt, n_steps,
                        n_steps_per_orbit, save_stride, nsave, w_out, w_final);
     return launch_status();
@@ -341,13 +351,8 @@ extern "C" int gamd_leapfrog_resume(const gamd_potential *pot, const double *w_h
     if (!pot || !w_half || !w_final || n_steps < 0) return GAMD_ERR_INVALID;
     if (N == 0) return GAMD_OK;
     const unsigned g = grid_for(N, LF_BLOCK);
-    const bool scf = pot->dev.has_scf;
-    const bool mw = pot->dev.layout == LAYOUT_MW;
-    const bool scf106 = pot->dev.layout == LAYOUT_SCF106;
-    auto kern = scf106 ? k_leapfrog<true, false, LAYOUT_SCF106, true>
-                : scf  ? k_leapfrog<true, false, LAYOUT_GENERIC, true>
-                : mw   ? k_leapfrog<false, false, LAYOUT_MW, true>
-                       : k_leapfrog<false, false, LAYOUT_GENERIC, true>;
+    auto kern = by_layout(
+        pot, [](auto scf, auto lay) { return k_leapfrog<scf.value, false, lay.value, true>; });
     hipLaunchKernelGGL(kern, dim3(g), dim3(LF_BLOCK), 0, as_stream(stream), pot->ddev, w_half,
                        (int64_t)N, dt, n_steps, n_steps_per_orbit, (int64_t)1, (int64_t)0,
                        (double *)nullptr, w_final);
@@ -379,13 +384,8 @@ extern "C" int gamd_leapfrog_stream(const gamd_potential *pot, const double *w0,
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int rc = GAMD_ERR_HIP;
-    const bool scf = pot->dev.has_scf;
-    const bool mw = pot->dev.layout == LAYOUT_MW;
-    const bool scf106 = pot->dev.layout == LAYOUT_SCF106;
-    auto run = scf106 ? stream_chunks<true, LAYOUT_SCF106>
-               : scf  ? stream_chunks<true, LAYOUT_GENERIC>
-               : mw   ? stream_chunks<false, LAYOUT_MW>
-                      : stream_chunks<false, LAYOUT_GENERIC>;
+    auto run =
+        by_layout(pot, [](auto scf, auto lay) { return stream_chunks<scf.value, lay.value>; });
     if (hipStreamCreateWithFlags(&c, hipStreamNonBlocking) != hipSuccess) goto done;
     if (hipEventCreateWithFlags(&comp, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&copied[0], hipEventDisableTiming) != hipSuccess ||
@@ -448,17 +448,9 @@ extern "C" int gamd_ruth4(const gamd_potential *pot, const double *w0, size_t N,
     const int64_t nsave = w_out ? n_steps / save_stride + 1 : 0;
     const unsigned g = grid_for(N, LF_BLOCK);
     hipStream_t s = as_stream(stream);
-    const bool scf = pot->dev.has_scf;
-    const bool mw = pot->dev.layout == LAYOUT_MW;
-    const bool scf106 = pot->dev.layout == LAYOUT_SCF106;
-    auto kern = w_out ? (scf106 ? k_ruth4<true, true, LAYOUT_SCF106>
-                         : scf  ? k_ruth4<true, true, LAYOUT_GENERIC>
-                         : mw   ? k_ruth4<false, true, LAYOUT_MW>
-                                : k_ruth4<false, true, LAYOUT_GENERIC>)
-                      : (scf106 ? k_ruth4<true, false, LAYOUT_SCF106>
-                         : scf  ? k_ruth4<true, false, LAYOUT_GENERIC>
-                         : mw   ? k_ruth4<false, false, LAYOUT_MW>
-                                : k_ruth4<false, false, LAYOUT_GENERIC>);
+    auto kern = by_layout(pot, [&](auto scf, auto lay) {
+        return w_out ? k_ruth4<scf.value, true, lay.value> : k_ruth4<scf.value, false, lay.value>;
+    });
     hipLaunchKernelGGL(kern, dim3(g), dim3(LF_BLOCK), 0, s, pot->ddev, w0, (int64_t)N, dt, n_steps,
                        save_stride, nsave, cf, w_out, w_final);
     return launch_status();

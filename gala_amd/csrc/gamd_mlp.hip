@@ -1183,7 +1183,7 @@ __global__ __launch_bounds__(256, 2) void k_surrogate_step(
 // the exact leapfrog bit for bit.  A kernel of its own keeps the SCF
 // evaluator's registers out of the network kernel.
 template <int LAY>
-__global__ __launch_bounds__(256) void k_surrogate_fallback(const DevPot *__restrict__ Pp,
+__global__ __launch_bounds__(64, scf_waves(LAY)) void k_surrogate_fallback(const DevPot *__restrict__ Pp,
                                                             double *__restrict__ wq,
                                                             double *__restrict__ vsync,
                                                             const int32_t *__restrict__ fb,
@@ -1334,8 +1334,8 @@ int gamd_surrogate_leapfrog_step(const float *theta, const uint16_t *wbf, const 
     int rc = launch_status();
     if (rc) return rc;
     auto fk = scf->dev.layout == LAYOUT_SCF106 ? k_surrogate_fallback<LAYOUT_SCF106>
-                                                : k_surrogate_fallback<LAYOUT_GENERIC>;
-    hipLaunchKernelGGL(fk, dim3(grid_for(N, 256)), dim3(256), 0, s, scf->ddev, w, vsync,
+                                                : k_surrogate_fallback<LAYOUT_SCF>;
+    hipLaunchKernelGGL(fk, dim3(grid_for(N, 64)), dim3(64), 0, s, scf->ddev, w, vsync,
                        fallback_step, (int64_t)N, dt, mode);
     return launch_status();
 }

@@ -11,6 +11,8 @@ using namespace gamd;
 
 namespace {
 
+constexpr unsigned EVAL_BLOCK = 256;
+
 // Fold parameter-only products into d[] (the same IEEE products gala forms
 // per call in builtin_potentials.cpp).
 void fold_component(DevComp &c) {
@@ -41,22 +43,68 @@ void fold_component(DevComp &c) {
     }
 }
 
-template <bool SCF>
-__global__ void k_value(const DevPot *__restrict__ Pp, const double *__restrict__ q, size_t N, double *__restrict__ out) {
+// the SCF table of one component (gamd_scf.hpp); gala's index is i = m +
+// (lmax+1)(l + (lmax+1) n) (bfe.cpp:160)
+void scf_table(const gamd_component &src, double *t) {
+    const int nmax = src.nmax, lmax = src.lmax;
+    for (int l = 0; l <= lmax; l++) {
+        const double a = 2.0 * l + 1.5;
+        for (int n = 0; n <= nmax; n++) {
+            *t++ = n + a - 1.0;
+            *t++ = n + 2.0 * a - 2.0;
+            *t++ = n > 0 ? 1.0 / n : 0.0;
+            *t++ = n + 2.0 * a - 1.0;
+            *t++ = n > 1 ? 1.0 / (n - 1) : 0.0;
+            for (int m = 0; m <= l; m++) {
+                const size_t gi = (size_t)m + (lmax + 1) * (l + (size_t)(lmax + 1) * n);
+                *t++ = src.S[gi];
+                if (m > 0) *t++ = src.T[gi];
+            }
+        }
+        *t++ = -sqrt((2.0 * l + 3.0) / (2.0 * l + 2.0));
+        for (int m = 0; m < l; m++) {
+            const double l2 = (double)l * l, m2 = (double)m * m;
+            *t++ = m == l - 1 ? sqrt(2.0 * m + 3.0) : sqrt((4.0 * l2 - 1.0) / (l2 - m2));
+            *t++ = m == l - 1 ? 0.0
+                              : sqrt(((l - 1.0) * (l - 1.0) - m2) /
+                                     (4.0 * (l - 1.0) * (l - 1.0) - 1.0));
+            *t++ = sqrt((2.0 * l + 1.0) / (2.0 * l - 1.0) * (double)(l - m) * (l + m));
+        }
+    }
+}
+
+// Phi of a potential of any layout
+template <bool SCF, int LAY>
+__device__ __forceinline__ double value_any(const DevPot &P, double x, double y, double z) {
+    const DevComp &c = P.c[0];
+    double phi, gx, gy, gz;
+    if (LAY == LAYOUT_SCF106)
+        scf_field<10, 6, true, false>(c.coef, c.p[0], c.p[1], c.p[2], 10, 6, x, y, z, phi, gx, gy,
+                                      gz);
+    else if (LAY == LAYOUT_SCF)
+        scf_field<-1, GAMD_SCF_MAX_LMAX, true, false>(c.coef, c.p[0], c.p[1], c.p[2], c.nmax,
+                                                      c.lmax, x, y, z, phi, gx, gy, gz);
+    else
+        phi = pot_value<SCF>(P, x, y, z);
+    return phi;
+}
+
+template <bool SCF, int LAY>
+__global__ __launch_bounds__(SCF ? 64 : EVAL_BLOCK, scf_waves(LAY)) void k_value(const DevPot *__restrict__ Pp, const double *__restrict__ q, size_t N, double *__restrict__ out) {
     const DevPot &P = *Pp;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < N;
          i += (size_t)gridDim.x * blockDim.x)
-        out[i] = pot_value<SCF>(P, q[i], q[N + i], q[2 * N + i]);
+        out[i] = value_any<SCF, LAY>(P, q[i], q[N + i], q[2 * N + i]);
 }
 
-template <bool SCF>
-__global__ void k_gradient(const DevPot *__restrict__ Pp, const double *__restrict__ q, size_t N,
+template <bool SCF, int LAY>
+__global__ __launch_bounds__(SCF ? 64 : EVAL_BLOCK, scf_waves(LAY)) void k_gradient(const DevPot *__restrict__ Pp, const double *__restrict__ q, size_t N,
                            double *__restrict__ g) {
     const DevPot &P = *Pp;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < N;
          i += (size_t)gridDim.x * blockDim.x) {
         double gx, gy, gz;
-        pot_grad<SCF>(P, q[i], q[N + i], q[2 * N + i], gx, gy, gz);
+        pot_grad_l<SCF, LAY>(P, q[i], q[N + i], q[2 * N + i], gx, gy, gz);
         g[i] = gx;
         g[N + i] = gy;
         g[2 * N + i] = gz;
@@ -64,15 +112,15 @@ __global__ void k_gradient(const DevPot *__restrict__ Pp, const double *__restri
 }
 
 template <bool SCF>
-__global__ void k_d2_dr2(const DevPot *__restrict__ Pp, const double *__restrict__ q, size_t N, double *__restrict__ out) {
+__global__ __launch_bounds__(SCF ? 64 : EVAL_BLOCK) void k_d2_dr2(const DevPot *__restrict__ Pp, const double *__restrict__ q, size_t N, double *__restrict__ out) {
     const DevPot &P = *Pp;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < N;
          i += (size_t)gridDim.x * blockDim.x)
         out[i] = pot_d2_dr2<SCF>(P, q[i], q[N + i], q[2 * N + i]);
 }
 
-template <bool SCF>
-__global__ void k_energy(const DevPot *__restrict__ Pp, const double *__restrict__ w, size_t N, double *__restrict__ out) {
+template <bool SCF, int LAY>
+__global__ __launch_bounds__(SCF ? 64 : EVAL_BLOCK, scf_waves(LAY)) void k_energy(const DevPot *__restrict__ Pp, const double *__restrict__ w, size_t N, double *__restrict__ out) {
     const DevPot &P = *Pp;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < N;
          i += (size_t)gridDim.x * blockDim.x) {
@@ -80,7 +128,7 @@ __global__ void k_energy(const DevPot *__restrict__ Pp, const double *__restrict
         // static_frame_hamiltonian (builtin_frames.cpp:8-16) then the
         // potential terms (chamiltonian.cpp:11-16)
         const double E = 0.5 * (px * px + py * py + pz * pz);
-        out[i] = E + pot_value<SCF>(P, w[i], w[N + i], w[2 * N + i]);
+        out[i] = E + value_any<SCF, LAY>(P, w[i], w[N + i], w[2 * N + i]);
     }
 }
 
@@ -120,7 +168,16 @@ __global__ void k_hessian(const DevPot *__restrict__ Pp, const double *__restric
     }
 }
 
-constexpr unsigned EVAL_BLOCK = 256;
+// threads per block: one wave where a point costs thousands of instructions,
+// so that some tens of thousands of points reach every SIMD
+unsigned field_block(const gamd_potential *pot) { return pot->dev.has_scf ? 64 : EVAL_BLOCK; }
+
+// the instance of a field kernel for a potential's layout
+#define GAMD_FIELD_KERNEL(k, pot)                                          \
+    ((pot)->dev.layout == LAYOUT_SCF106 ? k<true, LAYOUT_SCF106>           \
+     : (pot)->dev.layout == LAYOUT_SCF  ? k<true, LAYOUT_SCF>              \
+     : (pot)->dev.has_scf               ? k<true, LAYOUT_GENERIC>          \
+                                        : k<false, LAYOUT_GENERIC>)
 
 int check_eval(const gamd_potential *pot, const double *q, size_t N, const double *out) {
     if (!pot || (N > 0 && (!q || !out))) return GAMD_ERR_INVALID;
@@ -168,19 +225,8 @@ int gamd_potential_create(const gamd_component *components, int ncomponents,
             }
             c.nmax = src.nmax;
             c.lmax = src.lmax;
-            const int nmax = src.nmax, lmax = src.lmax;
-            const size_t nlm = (size_t)(lmax + 1) * (lmax + 2) / 2;
-            std::vector<double> packed(nlm * (nmax + 1) * 2);
-            // gala's index i = m + (lmax+1)(l + (lmax+1) n) (bfe.cpp:160) ->
-            // per l, per n, m = 0..l, (S, T) interleaved (scf_pack_index)
-            for (int l = 0; l <= lmax; l++)
-                for (int m = 0; m <= l; m++)
-                    for (int n = 0; n <= nmax; n++) {
-                        const size_t gi = (size_t)m + (lmax + 1) * (l + (size_t)(lmax + 1) * n);
-                        const size_t pi = (size_t)scf_pack_index(l, m, n, nmax);
-                        packed[2 * pi] = src.S[gi];
-                        packed[2 * pi + 1] = src.T[gi];
-                    }
+            std::vector<double> packed((size_t)scf_table_size(src.nmax, src.lmax));
+            scf_table(src, packed.data());
             void *d = nullptr;
             if (hipMalloc(&d, packed.size() * sizeof(double)) != hipSuccess) {
                 gamd_potential_destroy(pot);
@@ -201,9 +247,9 @@ int gamd_potential_create(const gamd_component *components, int ncomponents,
         pot->dev.c[1].type == GAMD_HERNQUIST && pot->dev.c[2].type == GAMD_MIYAMOTONAGAI &&
         pot->dev.c[3].type == GAMD_NFW)
         pot->dev.layout = LAYOUT_MW;
-    if (ncomponents == 1 && pot->dev.all_unshifted && pot->dev.c[0].type == GAMD_SCF &&
-        pot->dev.c[0].nmax == 10 && pot->dev.c[0].lmax == 6)
-        pot->dev.layout = LAYOUT_SCF106;
+    if (ncomponents == 1 && pot->dev.all_unshifted && pot->dev.c[0].type == GAMD_SCF)
+        pot->dev.layout = pot->dev.c[0].nmax == 10 && pot->dev.c[0].lmax == 6 ? LAYOUT_SCF106
+                                                                              : LAYOUT_SCF;
     // Kernels read the table through a restrict-qualified pointer: with a
     // wave-uniform component index these become scalar loads, where a by-value
     // kernel argument indexed by a runtime component number would be copied to
@@ -236,11 +282,9 @@ int gamd_potential_value(const gamd_potential *pot, double t, const double *q, s
                          double *out, void *stream) {
     int rc = check_eval(pot, q, N, out);
     if (rc || N == 0) return rc;
-    const unsigned g = grid_for(N, EVAL_BLOCK);
-    if (pot->dev.has_scf)
-        hipLaunchKernelGGL(k_value<true>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, q, N, out);
-    else
-        hipLaunchKernelGGL(k_value<false>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, q, N, out);
+    const unsigned b = field_block(pot);
+    hipLaunchKernelGGL(GAMD_FIELD_KERNEL(k_value, pot), dim3(grid_for(N, b)), dim3(b), 0,
+                       as_stream(stream), pot->ddev, q, N, out);
     return launch_status();
 }
 
@@ -248,11 +292,9 @@ int gamd_potential_gradient(const gamd_potential *pot, double t, const double *q
                             double *grad, void *stream) {
     int rc = check_eval(pot, q, N, grad);
     if (rc || N == 0) return rc;
-    const unsigned g = grid_for(N, EVAL_BLOCK);
-    if (pot->dev.has_scf)
-        hipLaunchKernelGGL(k_gradient<true>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, q, N, grad);
-    else
-        hipLaunchKernelGGL(k_gradient<false>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, q, N, grad);
+    const unsigned b = field_block(pot);
+    hipLaunchKernelGGL(GAMD_FIELD_KERNEL(k_gradient, pot), dim3(grid_for(N, b)), dim3(b), 0,
+                       as_stream(stream), pot->ddev, q, N, grad);
     return launch_status();
 }
 
@@ -278,11 +320,9 @@ int gamd_potential_d2_dr2(const gamd_potential *pot, double t, const double *q, 
                           double *out, void *stream) {
     int rc = check_eval(pot, q, N, out);
     if (rc || N == 0) return rc;
-    const unsigned g = grid_for(N, EVAL_BLOCK);
-    if (pot->dev.has_scf)
-        hipLaunchKernelGGL(k_d2_dr2<true>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, q, N, out);
-    else
-        hipLaunchKernelGGL(k_d2_dr2<false>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, q, N, out);
+    const unsigned b = field_block(pot);
+    hipLaunchKernelGGL(pot->dev.has_scf ? k_d2_dr2<true> : k_d2_dr2<false>, dim3(grid_for(N, b)),
+                       dim3(b), 0, as_stream(stream), pot->ddev, q, N, out);
     return launch_status();
 }
 
@@ -290,11 +330,9 @@ int gamd_hamiltonian_energy(const gamd_potential *pot, double t, const double *w
                             double *out, void *stream) {
     int rc = check_eval(pot, w, N, out);
     if (rc || N == 0) return rc;
-    const unsigned g = grid_for(N, EVAL_BLOCK);
-    if (pot->dev.has_scf)
-        hipLaunchKernelGGL(k_energy<true>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, w, N, out);
-    else
-        hipLaunchKernelGGL(k_energy<false>, dim3(g), dim3(EVAL_BLOCK), 0, as_stream(stream), pot->ddev, w, N, out);
+    const unsigned b = field_block(pot);
+    hipLaunchKernelGGL(GAMD_FIELD_KERNEL(k_energy, pot), dim3(grid_for(N, b)), dim3(b), 0,
+                       as_stream(stream), pot->ddev, w, N, out);
     return launch_status();
 }
 

@@ -56,6 +56,33 @@ def test_generic_layout_matches():
     assert np.max(np.abs(g - go) / np.linalg.norm(go, axis=0)) < 1e-11
 
 
+@pytest.mark.parametrize("nmax,lmax", [(0, 0), (1, 0), (2, 1), (10, 6), (10, 5), (0, 10), (3, 8),
+                                       (20, 10)])
+def test_every_size_matches_oracle(nmax, lmax):
+    """Smallest and largest tables, rows of one batch and of several, the
+    written-out size beside its neighbours; inner, outer and ordinary radii.
+    T_nl0 is not zero here and must not matter.  The bounds are those of
+    test_oracle_parity_benchmark_coefficients at ordinary radii."""
+    S, T = workloads.scf_coefficients(nmax, lmax, seed=nmax + lmax)
+    T[:, :, 0] = 0.25
+    pot = product_scf(1e12, 20.0, S, T)
+    orc = [O.scf(1e12, 20.0, S, T)]
+    rng = np.random.default_rng(nmax * 16 + lmax)
+    n = 333
+    q = rng.normal(size=(3, n))
+    q *= np.exp(rng.uniform(np.log(1.0), np.log(200.0), n)) / np.linalg.norm(q, axis=0)
+    v, vo = pot.energy(q), O.value(orc, q)
+    assert np.max(np.abs(v - vo) / np.max(np.abs(vo))) < 1e-12
+    g, go = pot.gradient(q), O.gradient(orc, q)
+    assert np.max(np.abs(g - go) / np.max(np.linalg.norm(go, axis=0))) < 1e-11
+    rho, rho_o = pot.density(q), O.density(orc, q)
+    assert np.max(np.abs(rho - rho_o) / np.max(np.abs(rho_o))) < 1e-11
+    # on the axis the value is finite and the gradient's angular part is 0 / 0
+    ax = np.array([[0.0, 0.0], [0.0, 0.0], [3.0, -40.0]])
+    np.testing.assert_allclose(pot.energy(ax), O.value(orc, ax), rtol=1e-11)
+    assert np.isnan(pot.gradient(ax)).all()
+
+
 def test_scf_leapfrog_and_dop853_parity():
     from gala_amd import _device as dev
     from gala_amd.integrate import dop853, leapfrog
