@@ -68,9 +68,10 @@ __global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_leapfrog(con
         y = y + hy * dt;
         z = z + hz * dt;
         pot_grad_l<SCF, LAY>(P, x, y, z, gx, gy, gz);
-        vx = hx - gx * dt / 2.0;
-        vy = hy - gy * dt / 2.0;
-        vz = hz - gz * dt / 2.0;
+        // hx - gx dt / 2 (the halving is exact)
+        vx = fma(-0.5, gx * dt, hx);
+        vy = fma(-0.5, gy * dt, hy);
+        vz = fma(-0.5, gz * dt, hz);
         hx = hx - gx * dt;
         hy = hy - gy * dt;
         hz = hz - gz * dt;
@@ -242,9 +243,10 @@ __global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_leapfrog_chu
         y = y + hy * dt;
         z = z + hz * dt;
         pot_grad_l<SCF, LAY>(P, x, y, z, gx, gy, gz);
-        vx = hx - gx * dt / 2.0;
-        vy = hy - gy * dt / 2.0;
-        vz = hz - gz * dt / 2.0;
+        // hx - gx dt / 2 (the halving is exact)
+        vx = fma(-0.5, gx * dt, hx);
+        vy = fma(-0.5, gy * dt, hy);
+        vz = fma(-0.5, gz * dt, hz);
         hx = hx - gx * dt;
         hy = hy - gy * dt;
         hz = hz - gz * dt;

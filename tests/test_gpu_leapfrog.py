@@ -196,3 +196,30 @@ def test_integrate_orbit_leapfrog_streams_to_host():
     orbit = Hamiltonian(mw_product()).integrate_orbit(w0, t=t, Integrator="leapfrog")
     wout, _ = leapfrog(mw_product(), w0, dt, 800)
     assert np.array_equal(orbit.w(), dev.to_host(wout))
+
+
+@pytest.mark.parametrize("r", [0.0, 1e-150, 1e-141, 1e-139, 1e-137, 1e-60, 1e-20, 0.1, 8.0, 1e3,
+                               1e39, 1e40, 1e41, 1e60])
+def test_milky_way_layout_at_extreme_radii(r):
+    """The straight-line Milky-Way evaluator shares one reciprocal of a product
+    of denominators, which leaves the range of a double below r ~ 1e-139 and
+    above r ~ 1e40 kpc and there gives way to the per-component forms: one
+    step's kick equals the one of the same four components evaluated by the
+    general loop (a NullPotential in front selects it) on both sides of either
+    end, alone and among orbits at ordinary radii.  Both evaluators are within
+    1e-13 of the reference's forms, so 4e-13 apart at most."""
+    from gala_amd import _device as dev
+    from gala_amd.integrate import leapfrog
+    from gala_amd.potential import CompositePotential, MilkyWayLikePotential, NullPotential
+    mw = MilkyWayLikePotential()
+    general = CompositePotential()
+    general["none"] = NullPotential()
+    for k, v in MilkyWayLikePotential().items():
+        general[k] = v
+    u = np.array([0.48, -0.6, 0.64])
+    w0 = np.zeros((6, 67))
+    w0[:3, 1:] = 8.0 * u[:, None]
+    w0[:3, 0] = w0[:3, 40] = r * u
+    a, b = (dev.to_host(leapfrog(p, w0, 1e-3, 1, save=False)[1]) for p in (mw, general))
+    np.testing.assert_allclose(a, b, rtol=4e-13, atol=0.0, equal_nan=True)
+    assert np.isfinite(a[:, 1:40]).all()
