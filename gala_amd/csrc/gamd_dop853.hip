@@ -664,12 +664,15 @@ struct WaveBodies {
 // over the system's 6 nb components in the order of the (6, nb) state
 // vector, component-major, as dop853.cpp:416-444 and :463-486 loop over it:
 // every lane stages its six squared terms in LDS, rounded as the reference
-// rounds sqr*sqr, and the 6 nb terms of each sum are then added in that order
-// by one wave (a workgroup of two or more waves gives the two sums to two
-// waves, which halves the serial chain of dependent adds each wave waits on;
-// a one-wave batch adds both), so the workgroup's lanes reach the same sums
+// rounds sqr*sqr, and the 6 nb terms of both sums are then added in that order
+// by the first wave (row_chains), so the workgroup's lanes reach the same sums
 // and take the same step decision.  Lanes past nb mirror orbit 0 of the batch
-// and stay out of the sums.
+// and stay out of the sums.  The serial chain of adds was what a batch waited
+// for longest: two waves, each with one chain fed from LDS term by term, took
+// 110 ms for 262,144 orbits in batches of 100 over 1 Gyr; one wave with both
+// chains, 16 terms to a register, takes 81.4 ms (8.2 -> 6.1 ms for 137 orbits,
+// two batches, over 500 Myr: there an attempt is about 17,000 cycles, 5,000 of
+// them this chain).
 template <bool SCF, int LAY>
 struct BatchLanes {
     static constexpr int NC = 6;
@@ -694,56 +697,62 @@ struct BatchLanes {
         }
         __syncthreads();
         if (nb > 64) {
-            // two or more waves: wave 0 adds the a-terms, wave 1 the b-terms,
-            // and they trade results through LDS
-            const int w = j >> 6;
-            if (w < 2) {
-                const double r = chain(w ? sb : sa, lds + w * n, n);
-                if ((j & 63) == 0) lds[2 * n + w] = r;
+            // two or more waves: the first adds, the others read its sums
+            if (__builtin_amdgcn_readfirstlane(j) < 64) {
+                const double r = row_chains(sa, sb, n);
+                if (j == 0) lds[2 * n] = r;
+                if (j == 16) lds[2 * n + 1] = r;
             }
             __syncthreads();
             sa = lds[2 * n];
             sb = lds[2 * n + 1];
             return;
         }
-        double xa = sa, xb = sb;
-        int i = 0;
-        // eight terms of each sum read ahead of their adds (the adds keep the
-        // reference's order; the reads of a block overlap one LDS latency)
-        constexpr int U = 8;
-        for (; i + U <= n; i += U) {
-            double ta[U], tb[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                ta[u] = lds[i + u];
-                tb[u] = lds[n + i + u];
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                xa += ta[u];
-                xb += tb[u];
-            }
-        }
-        for (; i < n; i++) {
-            xa += lds[i];
-            xb += lds[n + i];
-        }
-        sa = xa;
-        sb = xb;
+        const double r = row_chains(sa, sb, n);
+        sa = lane_bcast(r, 0);
+        sb = lane_bcast(r, 16);
     }
-    // x + t[0] + t[1] + ... + t[n - 1], added in that order
-    __device__ __forceinline__ static double chain(double x, const double *t, int n) {
-        int i = 0;
-        constexpr int U = 8;
-        for (; i + U <= n; i += U) {
-            double v[U];
+    // sa + the n a-terms in lane 0 and sb + the n b-terms in lane 16, each added
+    // one by one in order.  One wave does both: a row of 16 lanes holds 16
+    // terms at a time, the even rows a-terms and the odd rows b-terms, and 16
+    // multiply-adds by one (x + t exactly as an add rounds it) take them from
+    // lanes 0, 1, ... of their row (DPP row_newbcast) in turn.  Terms past the
+    // n count as zero, which changes no sum of squares.
+    __device__ __forceinline__ double row_chains(double sa, double sb, int n) const {
+        const int i = j & 15;
+        const bool odd = (j & 16) != 0;
+        const double *t = lds + (odd ? n : 0) + i;
+        double x = odd ? sb : sa;
+        // Four blocks are read ahead, so that no add waits for LDS: up to 63
+        // doubles past the terms, where the tableau lies.
+        double v[4];
 #pragma unroll
-            for (int u = 0; u < U; u++) v[u] = t[i + u];
+        for (int q = 0; q < 4; q++) v[q] = t[16 * q];
+        int k = 0;
+        for (; k + 64 <= n; k += 64) {
 #pragma unroll
-            for (int u = 0; u < U; u++) x += v[u];
+            for (int q = 0; q < 4; q++) {
+                add_row(x, v[q]);
+                v[q] = t[k + 64 + 16 * q];
+            }
         }
-        for (; i < n; i++) x += t[i];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (k + 16 * q < n) add_row(x, k + 16 * q + i < n ? v[q] : 0.0);
         return x;
+    }
+    // x += t of lane 0 of the row, then of lane 1, ..., lane 15.  (A DPP read
+    // of a register that a vector instruction has just written needs two
+    // waits: the s_nop.)
+    __device__ __forceinline__ static void add_row(double &x, double t) {
+        const double one = 1.0;
+#define GAMD_ADD(L) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #L " row_mask:0xf bank_mask:0xf\n"
+        asm("s_nop 1\n" GAMD_ADD(0) GAMD_ADD(1) GAMD_ADD(2) GAMD_ADD(3) GAMD_ADD(4) GAMD_ADD(5)
+                GAMD_ADD(6) GAMD_ADD(7) GAMD_ADD(8) GAMD_ADD(9) GAMD_ADD(10) GAMD_ADD(11)
+                    GAMD_ADD(12) GAMD_ADD(13) GAMD_ADD(14) GAMD_ADD(15)
+            : "+&v"(x)
+            : "v"(t), "v"(one));
+#undef GAMD_ADD
     }
     __device__ __forceinline__ double n() const { return 6.0 * (double)nb; }
     // dense sample s.oidx of the lane's orbit into w_out (6, n_out, N)

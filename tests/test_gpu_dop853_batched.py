@@ -112,6 +112,38 @@ def test_batched_final_states_and_stats(nbatch, n):
            max_gated=n // 20)
 
 
+@pytest.mark.parametrize("nbatch", [2, 5, 8, 11, 16, 21, 32, 43, 64, 65, 100, 128, 1024])
+def test_batch_sums_take_every_term(nbatch):
+    """The 6 nbatch terms of a batch's sums at the edges of the blocks of 16
+    and 64 they are added in (12 to 6144 terms; the last batch has 6), and of
+    one wave and several.  At a tolerance of 1e-5 a batch's truncation error
+    moves with its common step far more than rounding moves the states: the
+    bar is 100 times the oracle's one-ulp response (at least 1e-9), and one
+    term left out or counted twice, which the step sees as a tolerance
+    1/(12 nbatch) further off, has to move the oracle by ten times the bar."""
+    from gala_amd import _device as dev
+    from gala_amd import workloads
+    from gala_amd.integrate import dop853_batched
+    from tests.helpers import vcirc_oracle
+    orc = mw_oracle()
+    n, tol = 2 * nbatch + 1, 1e-5
+    w0 = np.ascontiguousarray(workloads.composite_leapfrog(vcirc_oracle(orc), n=2050,
+                                                           seed=21)[0][:, :n])
+    t = np.linspace(0.0, 200.0, 201)
+    ref, st_ref, _ = O.dop853(orc, w0, t, atol=tol, rtol=tol, nbatch=nbatch, save_all=False)
+    bar = np.maximum(1e-9, 100.0 * _sensitivity(orc, w0, t, nbatch, False, atol=tol, rtol=tol))
+    off = tol * (1.0 + 1.0 / (12 * nbatch))
+    moved = state_rel_err(O.dop853(orc, w0, t, atol=off, rtol=off, nbatch=nbatch,
+                                   save_all=False)[0], ref)
+    assert np.any(moved[:nbatch] > 10.0 * bar[:nbatch])
+    res = dop853_batched(mw_product(), w0, t[0], t[-1], t[1] - t[0], nbatch=nbatch, atol=tol,
+                         rtol=tol)
+    err = state_rel_err(dev.to_host(res["w_final"]), ref)
+    print(f"nbatch={nbatch}: max err {err.max():.3e}, at most {np.max(err / bar):.3e} of the bar")
+    assert np.array_equal(dev.to_host(res["status"]), st_ref)
+    assert np.all(err <= bar)
+
+
 def test_batched_generic_layout_and_hinit():
     """A potential outside the Milky-Way evaluator (generic component loop,
     shifted component), and h0 = 0 (Hairer's initial step over the batch,
