@@ -75,10 +75,8 @@ __device__ __forceinline__ double fma_const(double z, double k, double c) {
     return d;
 }
 
-// ln(2^e (1 + f)) from s = f / (2 + f)
-__device__ __forceinline__ double log_series(double s, int e) {
-    const double z = s * s;
-    const double z2 = z * z, z4 = z2 * z2, z8 = z4 * z4;
+// the series' polynomial in z = s^2 (z2 = z^2, ...)
+__device__ __forceinline__ double log_poly(double z, double z2, double z4, double z8) {
     const double p01 = fma(z, 0.3333333333333333, 1.0);
     const double p23 = fma_const(z, 0.14285714285714285, 0.2);
     const double p45 = fma_const(z, 0.09090909090909091, 0.1111111111111111);
@@ -88,10 +86,23 @@ __device__ __forceinline__ double log_series(double s, int e) {
     const double q03 = fma(z2, p23, p01);
     const double q47 = fma(z2, p67, p45);
     const double q8b = fma(z2, pab, p89);
-    const double P = fma(z8, q8b, fma(z4, q47, q03));
+    return fma(z8, q8b, fma(z4, q47, q03));
+}
+
+// ln(2^e (1 + f)) from s = f / (2 + f)
+template <class Poly>
+__device__ __forceinline__ double log_series(double s, int e, const Poly &poly) {
+    const double z = s * s;
+    const double z2 = z * z, z4 = z2 * z2, z8 = z4 * z4;
+    const double P = poly(z, z2, z4, z8);
     const double ed = (double)e;
     const double lm = (s + s) * P;
     return fma(ed, 0.6931471803691238, fma(ed, 1.9082149292705877e-10, lm));
+}
+__device__ __forceinline__ double log_series(double s, int e) {
+    return log_series(s, e, [](double z, double z2, double z4, double z8) {
+        return log_poly(z, z2, z4, z8);
+    });
 }
 
 __device__ __forceinline__ double log_fast(double x) {
@@ -569,29 +580,50 @@ __device__ __forceinline__ void mw_grad_extreme(const DevPot &P, double x, doubl
 // issue, 96 % busy) 3.98 -> 3.76 ms; the uneven DOP853 launch over 1,048,576
 // orbits, its longest orbit's 23,800 attempts in a row, 129 -> 115 ms.  The same
 // operations on the same values, so the same results bit for bit.
-__device__ __forceinline__ void mw_grad(const DevPot &P, double x, double y, double z,
-                                        double &gx, double &gy, double &gz) {
-    const DevComp &h1 = P.c[0], &h2 = P.c[1], &mn = P.c[2], &nf = P.c[3];
-    const double gmn = nf.d[0] * nf.d[1];
+struct MwFactors {
+    double f1, f2, f3, f3z, f4;  // of q: nucleus, bulge, disk (and its z), halo
+    bool extreme;                // they are not to be used
+};
+struct MwConstants {
+    double m1, c1, m2, c2;    // nucleus and bulge: G m, c
+    double m3, a3, b3sq;      // disk: G m, a, b^2
+    double m4, irs4;          // halo: G m, 1 / r_s
+    __device__ __forceinline__ explicit MwConstants(const DevPot &P)
+        : m1(P.c[0].d[0]), c1(P.c[0].d[1]), m2(P.c[1].d[0]), c2(P.c[1].d[1]), m3(P.c[2].d[0]),
+          a3(P.c[2].d[1]), b3sq(P.c[2].d[2]), m4(P.c[3].d[0] * P.c[3].d[1]), irs4(P.c[3].d[3]) {}
+};
+// how a lane evaluates them: all of it alone
+struct MwAlone {
+    __device__ __forceinline__ static void rsqrt_pair(double a, double b, double &ra, double &rb) {
+        ra = rsqrt_nr(a);
+        rb = rsqrt_nr(b);
+    }
+    __device__ __forceinline__ double operator()(double z, double z2, double z4, double z8) const {
+        return log_poly(z, z2, z4, z8);
+    }
+};
+template <class Lanes>
+__device__ __forceinline__ MwFactors mw_factors(const MwConstants &m, const Lanes &lanes, double x,
+                                                double y, double z) {
     const double R2 = x * x + y * y;
     const double r2 = R2 + z * z;
     // |q|, 1/|q|^3, sqrt(z^2 + b^2), its inverse and D^(-3/2) from three
     // reciprocal square roots instead of three correctly rounded roots and
     // their divides
-    const double ir = rsqrt_nr(r2);
+    const double s2 = z * z + m.b3sq;
+    double ir, isz;
+    lanes.rsqrt_pair(r2, s2, ir, isz);
     const double r = r2 * ir;
     const double ir3 = ir * ir * ir;
-    const double s2 = z * z + mn.d[2];
-    const double isz = rsqrt_nr(s2);
     const double sqrtz = s2 * isz;
-    const double zd = mn.d[1] + sqrtz;
+    const double zd = m.a3 + sqrtz;
     const double D = R2 + zd * zd;
     const double iD = rsqrt_nr(D);
-    const double f3 = mn.d[0] * (iD * iD * iD);
-    const double f3z = 1.0 + mn.d[1] * isz;
+    const double f3 = m.m3 * (iD * iD * iD);
+    const double f3z = 1.0 + m.a3 * isz;
     // NFW in the equivalent form G m / r^3 (log(1+u) - u/(1+u)), u = r / r_s
     // (v_h2 / u^3 / r_s^2 = G m / r^3)
-    const double u = r * nf.d[3];  // d[3] = 1 / r_s
+    const double u = r * m.irs4;
     const double opu = 1.0 + u;
     double lf;
     int le;
@@ -600,8 +632,8 @@ __device__ __forceinline__ void mw_grad(const DevPot &P, double x, double y, dou
     // The remaining denominators -- the two Hernquist ones, 1 + u and the
     // log's 2 + f -- share one reciprocal (batched inversion: invert the
     // product, peel the factors off with multiplies).
-    const double rc1 = r + h1.d[1];
-    const double rc2 = r + h2.d[1];
+    const double rc1 = r + m.c1;
+    const double rc2 = r + m.c2;
     const double d1 = rc1 * rc1 * r, d2 = rc2 * rc2 * r;
     const double p12 = d1 * d2;
     const double p3 = p12 * opu;
@@ -611,26 +643,58 @@ __device__ __forceinline__ void mw_grad(const DevPot &P, double x, double y, dou
     const double inv3 = inv * tf;
     const double inv2 = inv3 * opu;
     const double i4 = inv3 * p12;
-    const double f1 = h1.d[0] * (inv2 * d2);
-    const double f2 = h2.d[0] * (inv2 * d1);
-    const double lg = log_series(slog, le);
-    const double f4 = gmn * (lg - u * i4) * ir3;
+    const double f1 = m.m1 * (inv2 * d2);
+    const double f2 = m.m2 * (inv2 * d1);
+    const double lg = log_series(slog, le, lanes);
+    const double f4 = m.m4 * (lg - u * i4) * ir3;
+    // p's high word outside [1e-280's, 1e280's): one compare of integers
+    constexpr unsigned lo = 0x05CD0B15u, hi = 0x7A11A0FCu;
+    return {f1, f2, f3, f3z, f4, (unsigned)__double2hiint(p) - lo >= hi - lo};
+}
+
+__device__ __forceinline__ void mw_grad(const DevPot &P, double x, double y, double z,
+                                        double &gx, double &gy, double &gz) {
+    const MwFactors m = mw_factors(MwConstants(P), MwAlone{}, x, y, z);
     gx = 0.0;
     gy = 0.0;
     gz = 0.0;
-    gx += f1 * x;
-    gy += f1 * y;
-    gz += f1 * z;
-    gx += f2 * x;
-    gy += f2 * y;
-    gz += f2 * z;
-    gx += f3 * x;
-    gy += f3 * y;
-    gz += f3 * z * f3z;
-    gx += f4 * x;
-    gy += f4 * y;
-    gz += f4 * z;
-    if (__builtin_expect(!(p > 1e-280 && p < 1e280), 0)) mw_grad_extreme(P, x, y, z, gx, gy, gz);
+    gx += m.f1 * x;
+    gy += m.f1 * y;
+    gz += m.f1 * z;
+    gx += m.f2 * x;
+    gy += m.f2 * y;
+    gz += m.f2 * z;
+    gx += m.f3 * x;
+    gy += m.f3 * y;
+    gz += m.f3 * z * m.f3z;
+    gx += m.f4 * x;
+    gy += m.f4 * y;
+    gz += m.f4 * z;
+    if (__builtin_expect(__any(m.extreme), 0))
+        if (m.extreme) mw_grad_extreme(P, x, y, z, gx, gy, gz);
+}
+
+// mw_grad along one axis (0, 1, 2), q being the position along it: for lanes
+// that hold one component each
+template <class Lanes>
+__device__ __forceinline__ double mw_grad_along(const DevPot &P, const MwConstants &mc,
+                                                const Lanes &lanes, double x, double y, double z,
+                                                int axis, double q) {
+    const MwFactors m = mw_factors(mc, lanes, x, y, z);
+    double g = 0.0;
+    g += m.f1 * q;
+    g += m.f2 * q;
+    double gr = g, gz = g;
+    gr += m.f3 * q;
+    gz += m.f3 * q * m.f3z;
+    g = axis == 2 ? gz : gr;
+    g += m.f4 * q;
+    if (__builtin_expect(__any(m.extreme), 0)) {
+        double ex, ey, ez;
+        mw_grad_extreme(P, x, y, z, ex, ey, ez);
+        if (m.extreme) g = axis == 2 ? ez : (axis == 1 ? ey : ex);
+    }
+    return g;
 }
 
 // grad Phi with the layout chosen at compile time (LAYOUT_GENERIC reads the

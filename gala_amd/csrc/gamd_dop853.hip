@@ -127,11 +127,10 @@ __device__ double hinit(const DevPot &P, double x, const double *y, double posne
 //   NC = 6: one lane owns one orbit (the bulk of the run);
 //   NC = 1: the "wide tail": once the queue is drained and a wave holds at
 //           most four unfinished orbits, each orbit is spread over one DPP
-//           row of 16 lanes, lane c of the row holding component c % 6 (lanes
-//           12..15 duplicate components 3..5).  The stage combinations, error
-//           terms and dense updates then cost one component's arithmetic
-//           instead of six; every lane of the row evaluates the force at the
-//           row's broadcast position.  Sums over components are formed from
+//           row of 16 lanes, each lane holding one component (WideRow).  The
+//           stage combinations, error terms and dense updates then cost one
+//           component's arithmetic instead of six; every lane of the row
+//           evaluates the force at the row's broadcast position.  Sums over components are formed from
 //           broadcast terms in the one-lane order, so both layouts produce
 //           bit-identical results.
 // The tail matters because the uneven workload's longest orbits need ~5x the
@@ -141,20 +140,21 @@ constexpr int WIDE_ROW = 16;   // lanes per orbit in the wide tail (one DPP row)
 constexpr int WIDE_ORBITS = 4; // orbits per wave in the wide tail
 constexpr int QUAD_ORBITS = 16; // orbits per wave in the quad tail (one per 4-lane quad)
 
+// llvm.amdgcn.update.dpp on a double: one v_mov_b64_dpp (the builtin takes 32 bits)
+__device__ double dpp_f64(double old, double v, int ctrl, int row_mask, int bank_mask,
+                          bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.f64");
+
 template <int SRC>
 __device__ __forceinline__ double row_bcast(double v) {
     // DPP row_newbcast:SRC: every lane of a 16-lane row reads lane SRC of the
-    // row (every lane has a source in its row, so no "old" value is needed)
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + SRC, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + SRC, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
+    // row (every lane has a source in its row, so the zero is not used)
+    return dpp_f64(0.0, v, 0x150 + SRC, 0xF, 0xF, true);
 }
 
-// DPP row_shl:3: lane i of a row reads lane i + 3 (lanes 13..15 keep their own)
-__device__ __forceinline__ double row_shl3(double v) {
-    const int lo0 = __double2loint(v), hi0 = __double2hiint(v);
-    const int lo = __builtin_amdgcn_update_dpp(lo0, lo0, 0x103, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(hi0, hi0, 0x103, 0xF, 0xF, false);
+// DPP row_half_mirror: lane i of 8 reads lane 7 - i
+__device__ __forceinline__ double half_mirror(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x141, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x141, 0xF, 0xF, false);
     return __hiloint2double(hi, lo);
 }
 
@@ -335,26 +335,278 @@ struct OneLaneTab : OneLane<SCF, LAY> {
     const double *tab;
 };
 
-// one orbit per 16-lane row, lane c holding component comp
-template <bool SCF, int LAY>
+// The tableau as one array (A 16x16, D 4x16, B, E5, BHH), for layouts that
+// read it from LDS (a layout declares LDS_TABLEAU = true and a member `tab`
+// pointing at an LDS copy of kTableau).
+constexpr int TAB_OFS_A = 0, TAB_OFS_D = 256, TAB_OFS_B = 320, TAB_OFS_E5 = 332,
+              TAB_OFS_BHH = 345, TAB_WORDS = 358;
+struct TableauWords {
+    double w[TAB_WORDS];
+};
+constexpr TableauWords make_tableau() {
+    TableauWords t{};
+    for (int i = 0; i < 16; i++)
+        for (int j = 0; j < 16; j++) t.w[TAB_OFS_A + i * 16 + j] = T::A[i][j];
+    for (int i = 0; i < 4; i++)
+        for (int j = 0; j < 16; j++) t.w[TAB_OFS_D + i * 16 + j] = T::D[i][j];
+    for (int k = 0; k < 12; k++) t.w[TAB_OFS_B + k] = T::B[k];
+    for (int k = 0; k < 13; k++) t.w[TAB_OFS_E5 + k] = T::E5[k];
+    for (int k = 0; k < 13; k++) t.w[TAB_OFS_BHH + k] = T::BHH[k];
+    return t;
+}
+__constant__ TableauWords kTableau = make_tableau();
+
+// Linear combinations of derivatives with entries K... of TableauWords.
+template <int... K>
+struct Entries {};
+template <int I, int... J>
+using EntriesA = Entries<(TAB_OFS_A + I * 16 + J)...>;
+template <int I, int... J>
+using EntriesD = Entries<(TAB_OFS_D + I * 16 + J)...>;
+template <int... J>
+using EntriesB = Entries<(TAB_OFS_B + J)...>;
+template <int... J>
+using EntriesE5 = Entries<(TAB_OFS_E5 + J)...>;
+template <int... J>
+using EntriesBHH = Entries<(TAB_OFS_BHH + J)...>;
+
+// The tableau spread over the lanes of a 16-lane row: lane i holds entry
+// 16 q + i of the list below in register pair q, and a multiply-add takes it
+// from there (DPP row_newbcast), so that a term of a combination is one
+// instruction.  As literals the entries of an attempt took ~240 scalar moves
+// and 50 reloads of spilled scalars, of ~2,090 instructions.  The terms of one
+// combination lie in one register pair, in the order they are added.
+constexpr int ROW_REGS = 5, ROW_REGS_DENSE = 10;
+struct RowTableau {
+    int ofs[16 * ROW_REGS_DENSE];   // into TableauWords, -1 for none
+    double w[16 * ROW_REGS_DENSE];  // its value; BHH negated (it is subtracted)
+};
+template <int... K>
+constexpr int row_put(RowTableau &t, int at, Entries<K...>) {
+    const int k[] = {K...};
+    const TableauWords all = make_tableau();
+    for (int i = 0; i < (int)sizeof...(K); i++) {
+        t.ofs[at + i] = k[i];
+        t.w[at + i] = k[i] >= TAB_OFS_BHH ? -all.w[k[i]] : all.w[k[i]];
+    }
+    return at + (int)sizeof...(K);
+}
+constexpr RowTableau make_row_tableau() {
+    RowTableau t{};
+    for (int i = 0; i < 16 * ROW_REGS_DENSE; i++) t.ofs[i] = -1;
+    int at = row_put(t, 0, EntriesA<2, 0, 1>{});
+    at = row_put(t, at, EntriesA<3, 0, 2>{});
+    at = row_put(t, at, EntriesA<4, 0, 2, 3>{});
+    at = row_put(t, at, EntriesA<5, 0, 3, 4>{});
+    row_put(t, at, EntriesA<6, 0, 3, 4, 5>{});
+    at = row_put(t, 16, EntriesA<7, 0, 3, 4, 5, 6>{});
+    at = row_put(t, at, EntriesA<8, 0, 3, 4, 5, 6, 7>{});
+    at = row_put(t, at, EntriesBHH<0, 8, 11>{});
+    row_put(t, at, EntriesA<1, 0>{});
+    at = row_put(t, 32, EntriesA<9, 0, 3, 4, 5, 6, 7, 8>{});
+    row_put(t, at, EntriesA<10, 0, 3, 4, 5, 6, 7, 8, 9>{});
+    at = row_put(t, 48, EntriesA<11, 0, 3, 4, 5, 6, 7, 8, 9, 10>{});
+    row_put(t, at, EntriesD<0, 12, 13, 14, 15>{});
+    at = row_put(t, 64, EntriesB<0, 5, 6, 7, 8, 9, 10, 11>{});
+    row_put(t, at, EntriesE5<0, 5, 6, 7, 8, 9, 10, 11>{});
+    at = row_put(t, 80, EntriesA<13, 0, 6, 7, 8, 9, 10, 11, 12>{});
+    row_put(t, at, EntriesA<14, 0, 5, 6, 7, 10, 11, 12, 13>{});
+    at = row_put(t, 96, EntriesA<15, 0, 5, 6, 7, 8, 12, 13, 14>{});
+    row_put(t, at, EntriesD<0, 0, 5, 6, 7, 8, 9, 10, 11>{});
+    at = row_put(t, 112, EntriesD<1, 0, 5, 6, 7, 8, 9, 10, 11>{});
+    row_put(t, at, EntriesD<2, 0, 5, 6, 7, 8, 9, 10, 11>{});
+    at = row_put(t, 128, EntriesD<3, 0, 5, 6, 7, 8, 9, 10, 11>{});
+    at = row_put(t, at, EntriesD<1, 12, 13, 14, 15>{});
+    row_put(t, at, EntriesD<2, 12, 13, 14, 15>{});
+    row_put(t, 144, EntriesD<3, 12, 13, 14, 15>{});
+    return t;
+}
+constexpr RowTableau ROW_TABLEAU = make_row_tableau();
+__constant__ RowTableau kRowTableau = make_row_tableau();
+// where the combination K... starts; -1 unless all of it follows, in one register pair
+template <int... K>
+constexpr int row_slot(Entries<K...>) {
+    const int k[] = {K...}, n = (int)sizeof...(K);
+    for (int at = 0; at + n <= 16 * ROW_REGS_DENSE; at++) {
+        bool same = at / 16 == (at + n - 1) / 16;
+        for (int i = 0; i < n; i++) same = same && ROW_TABLEAU.ofs[at + i] == k[i];
+        if (same) return at;
+    }
+    return -1;
+}
+
+// t_L a + t_(L+1) b + ..., t_i the value of t in lane i of the row, rounded as
+// the expression over scalars is: the second product first, then one
+// multiply-add a term, in order.  (A DPP read of a register that a vector
+// instruction has just written needs two waits: the s_nop.)
+#define GAMD_TERM(K, I) \
+    "v_fmac_f64_dpp %0, %1, %" #K " row_newbcast:%" #I " row_mask:0xf bank_mask:0xf\n"
+#define GAMD_TERMS2 \
+    "s_nop 1\nv_mov_b64_dpp %0, %1 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n" \
+    "v_mul_f64 %0, %0, %12\n" GAMD_TERM(11, 2)
+#define GAMD_TERMS3 GAMD_TERMS2 GAMD_TERM(13, 4)
+#define GAMD_TERMS4 GAMD_TERMS3 GAMD_TERM(14, 5)
+#define GAMD_TERMS5 GAMD_TERMS4 GAMD_TERM(15, 6)
+#define GAMD_TERMS6 GAMD_TERMS5 GAMD_TERM(16, 7)
+#define GAMD_TERMS7 GAMD_TERMS6 GAMD_TERM(17, 8)
+#define GAMD_TERMS8 GAMD_TERMS7 GAMD_TERM(18, 9)
+#define GAMD_TERMS9 GAMD_TERMS8 GAMD_TERM(19, 10)
+#define GAMD_LANES \
+    "n"(L), "n"(L + 1), "n"(L + 2), "n"(L + 3), "n"(L + 4), "n"(L + 5), "n"(L + 6), "n"(L + 7), \
+        "n"(L + 8)
+template <int L, class... V>
+__device__ __forceinline__ double row_lin(double t, V... v) {
+    const double k[] = {v...};
+    constexpr int N = (int)sizeof...(V);
+    static_assert(N >= 2 && N <= 9, "2 to 9 terms");
+    double r;
+    if constexpr (N == 2)
+        asm(GAMD_TERMS2 : "=&v"(r) : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]));
+    else if constexpr (N == 3)
+        asm(GAMD_TERMS3 : "=&v"(r) : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]));
+    else if constexpr (N == 4)
+        asm(GAMD_TERMS4 : "=&v"(r)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]));
+    else if constexpr (N == 5)
+        asm(GAMD_TERMS5 : "=&v"(r)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]));
+    else if constexpr (N == 6)
+        asm(GAMD_TERMS6 : "=&v"(r)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]),
+              "v"(k[5]));
+    else if constexpr (N == 7)
+        asm(GAMD_TERMS7 : "=&v"(r)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]),
+              "v"(k[5]), "v"(k[6]));
+    else if constexpr (N == 8)
+        asm(GAMD_TERMS8 : "=&v"(r)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]),
+              "v"(k[5]), "v"(k[6]), "v"(k[7]));
+    else
+        asm(GAMD_TERMS9 : "=&v"(r)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "v"(k[4]),
+              "v"(k[5]), "v"(k[6]), "v"(k[7]), "v"(k[8]));
+    return r;
+}
+// acc + t_L a + t_(L+1) b + ..., one multiply-add a term, in order
+template <int L, class... V>
+__device__ __forceinline__ double row_add(double t, double acc, V... v) {
+    const double k[] = {v...};
+    constexpr int N = (int)sizeof...(V);
+    static_assert(N == 3 || N == 4, "3 or 4 terms");
+    if constexpr (N == 3)
+        asm("s_nop 1\n" GAMD_TERM(11, 2) GAMD_TERM(12, 3) GAMD_TERM(13, 4)
+            : "+&v"(acc)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]));
+    else
+        asm("s_nop 1\n" GAMD_TERM(11, 2) GAMD_TERM(12, 3) GAMD_TERM(13, 4) GAMD_TERM(14, 5)
+            : "+&v"(acc)
+            : "v"(t), GAMD_LANES, "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]));
+    return acc;
+}
+#undef GAMD_TERM
+#undef GAMD_TERMS2
+#undef GAMD_TERMS3
+#undef GAMD_TERMS4
+#undef GAMD_TERMS5
+#undef GAMD_TERMS6
+#undef GAMD_TERMS7
+#undef GAMD_TERMS8
+#undef GAMD_TERMS9
+#undef GAMD_LANES
+
+// The Milky-Way evaluator (mw_factors) on a 16-lane row whose lanes 0 to 7
+// use its result: the two reciprocal roots that do not wait for each other are
+// one, of r^2 in the lower and of z^2 + b^2 in the upper half, and the log's
+// polynomial is one chain of three lanes' coefficients instead of three.  The
+// same operations on the same values; a wave alone on its SIMD waits for the
+// issue of every instruction, of which an evaluation loses 8 in 117.
+struct RowMw {
+    MwConstants m;
+    double lo0, lo1, hi0, hi1;  // lane i: the i-th third of log_poly's coefficients
+    bool upper;
+    __device__ __forceinline__ RowMw(const DevPot &P, int lane) : m(P), upper(lane >= 8) {
+        lo0 = lane == 0 ? 1.0 : (lane == 1 ? 0.1111111111111111 : 0.058823529411764705);
+        lo1 = lane == 0 ? 0.3333333333333333
+                        : (lane == 1 ? 0.09090909090909091 : 0.05263157894736842);
+        hi0 = lane == 0 ? 0.2 : (lane == 1 ? 0.07692307692307693 : 0.047619047619047616);
+        hi1 = lane == 0 ? 0.14285714285714285
+                        : (lane == 1 ? 0.06666666666666667 : 0.043478260869565216);
+        // kept in vector registers: as scalars they were read again from
+        // memory, with a wait each, in every attempt
+        asm volatile("" : "+v"(m.m1), "+v"(m.c1), "+v"(m.m2), "+v"(m.c2), "+v"(m.m3), "+v"(m.a3),
+                     "+v"(m.b3sq), "+v"(m.m4), "+v"(m.irs4));
+        asm volatile("" : "+v"(lo0), "+v"(lo1), "+v"(hi0), "+v"(hi1));
+    }
+    __device__ __forceinline__ void rsqrt_pair(double a, double b, double &ra, double &rb) const {
+        ra = rsqrt_nr(upper ? b : a);
+        rb = row_bcast<8>(ra);
+    }
+    __device__ __forceinline__ double operator()(double z, double z2, double z4, double z8) const {
+        const double q = fma(z2, fma(z, hi1, hi0), fma(z, lo1, lo0));
+        double r;
+        asm("s_nop 1\n"
+            "v_mov_b64_dpp %0, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f64_dpp %0, %1, %3 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+            : "=&v"(r)
+            : "v"(q), "v"(z4), "v"(z8));
+        return r;
+    }
+};
+struct NoRowMw {
+    __device__ __forceinline__ NoRowMw(const DevPot &, int) {}
+};
+
+// one orbit per 16-lane row.  Lanes 0, 1, 2 hold x, y, z and lanes 7, 6, 5 the
+// velocities along them (lanes 3 and 4 mirror 2 and 5), so that a lane's
+// partner along its axis is the mirror image in its half of the row; a lane
+// needs only the gradient along its own axis.  Lanes 8 to 15 start as copies
+// of lanes 0 to 7 and help with the force; nothing reads their state.
+// An attempt of a wave alone on its SIMD costs the issue of its ~1,700
+// instructions (2,090 with the tableau as literals, three gradient components
+// and the force in one lane): the uneven launch over 1,048,576 orbits, which
+// lasts as long as its longest orbits' 25,700 attempts, 115.8 -> 91.2 ms.
+template <bool SCF, int LAY, bool DENSE>
 struct WideRow {
     static constexpr int NC = 1;
+    static constexpr bool ROW_TABLEAU = true;
     int comp;
-    bool writes;  // lanes 0..5 of the row store the dense samples
+    bool writes;  // lanes 0, 1, 2, 5, 6, 7 of the row store the dense samples
+    double tab[DENSE ? ROW_REGS_DENSE : ROW_REGS];
+    typename std::conditional<LAY == LAYOUT_MW, RowMw, NoRowMw>::type mw;
+    __device__ __forceinline__ static int comp_of(int lane) {
+        const int i = lane & 7;
+        return i < 3 ? i : (i == 3 ? 2 : (i == 4 ? 5 : 10 - i));
+    }
+    __device__ __forceinline__ static bool writes_of(int lane) {
+        return lane < 8 && lane != 3 && lane != 4;
+    }
+    __device__ __forceinline__ WideRow(const DevPot &P, int lane)
+        : comp(comp_of(lane)), writes(writes_of(lane)), mw(P, lane) {
+#pragma unroll
+        for (int q = 0; q < (DENSE ? ROW_REGS_DENSE : ROW_REGS); q++)
+            tab[q] = kRowTableau.w[16 * q + lane];
+    }
     __device__ __forceinline__ void rhs(const DevPot &P, const double (&y)[1], double (&f)[1]) const {
         const double qx = row_bcast<0>(y[0]), qy = row_bcast<1>(y[0]), qz = row_bcast<2>(y[0]);
-        const double vp = row_shl3(y[0]);  // the velocity partner of components 0..2
-        double gx, gy, gz;
-        pot_grad_l<SCF, LAY>(P, qx, qy, qz, gx, gy, gz);
-        const double g = comp == 3 ? gx : (comp == 4 ? gy : gz);
-        f[0] = comp < 3 ? vp : -g;
+        const double partner = half_mirror(y[0]);
+        double g;
+        if constexpr (LAY == LAYOUT_MW) {
+            g = mw_grad_along(P, mw.m, mw, qx, qy, qz, comp - 3, partner);
+        } else {
+            double gx, gy, gz;
+            pot_grad_l<SCF, LAY>(P, qx, qy, qz, gx, gy, gz);
+            g = comp == 3 ? gx : (comp == 4 ? gy : gz);
+        }
+        f[0] = comp < 3 ? partner : -g;
     }
     __device__ __forceinline__ static void all6(const double (&v)[1], double (&o)[6]) {
         o[0] = row_bcast<0>(v[0]);
         o[1] = row_bcast<1>(v[0]);
         o[2] = row_bcast<2>(v[0]);
-        o[3] = row_bcast<3>(v[0]);
-        o[4] = row_bcast<4>(v[0]);
+        o[3] = row_bcast<7>(v[0]);
+        o[4] = row_bcast<6>(v[0]);
         o[5] = row_bcast<5>(v[0]);
     }
     __device__ __forceinline__ void sums(const double (&a)[1], const double (&b)[1], double &sa,
@@ -827,27 +1079,6 @@ struct has_windows<S, decltype((void)S::WINDOWS)> {
     static constexpr bool value = S::WINDOWS;
 };
 
-// The tableau as one array (A 16x16, D 4x16, B, E5, BHH), for layouts that
-// read it from LDS (a layout declares LDS_TABLEAU = true and a member `tab`
-// pointing at an LDS copy of kTableau).
-constexpr int TAB_OFS_A = 0, TAB_OFS_D = 256, TAB_OFS_B = 320, TAB_OFS_E5 = 332,
-              TAB_OFS_BHH = 345, TAB_WORDS = 358;
-struct TableauWords {
-    double w[TAB_WORDS];
-};
-constexpr TableauWords make_tableau() {
-    TableauWords t{};
-    for (int i = 0; i < 16; i++)
-        for (int j = 0; j < 16; j++) t.w[TAB_OFS_A + i * 16 + j] = T::A[i][j];
-    for (int i = 0; i < 4; i++)
-        for (int j = 0; j < 16; j++) t.w[TAB_OFS_D + i * 16 + j] = T::D[i][j];
-    for (int k = 0; k < 12; k++) t.w[TAB_OFS_B + k] = T::B[k];
-    for (int k = 0; k < 13; k++) t.w[TAB_OFS_E5 + k] = T::E5[k];
-    for (int k = 0; k < 13; k++) t.w[TAB_OFS_BHH + k] = T::BHH[k];
-    return t;
-}
-__constant__ TableauWords kTableau = make_tableau();
-
 template <class S, class = void>
 struct lds_tableau {
     static constexpr bool value = false;
@@ -857,12 +1088,61 @@ struct lds_tableau<S, decltype((void)S::LDS_TABLEAU)> {
     static constexpr bool value = S::LDS_TABLEAU;
 };
 
-template <class Sys>
-__device__ __forceinline__ double tab_entry(const Sys &sys, int ofs, int k, double c) {
-    if constexpr (lds_tableau<Sys>::value)
-        return sys.tab[ofs + k];
-    else
+template <class S, class = void>
+struct row_tableau {
+    static constexpr bool value = false;
+};
+template <class S>
+struct row_tableau<S, decltype((void)S::ROW_TABLEAU)> {
+    static constexpr bool value = S::ROW_TABLEAU;
+};
+
+constexpr TableauWords TABLEAU = make_tableau();
+
+// tableau entry K
+template <int K, class Sys>
+__device__ __forceinline__ double tab_entry(const Sys &sys, int ofs) {
+    constexpr double c = TABLEAU.w[K];
+    if constexpr (row_tableau<Sys>::value) {
+        constexpr int at = row_slot(Entries<K>{});
+        return row_bcast<at % 16>(sys.tab[at / 16]);
+    } else if constexpr (lds_tableau<Sys>::value) {
+        return sys.tab[ofs + K];
+    } else {
         return c;
+    }
+}
+
+// the sum of the entries K... times v..., in order
+template <class Sys, int... K, class... V>
+__device__ __forceinline__ double lin(const Sys &sys, int ofs, Entries<K...> e, V... v) {
+    if constexpr (row_tableau<Sys>::value) {
+        constexpr int at = row_slot(Entries<K...>{});
+        static_assert(at >= 0, "not in the row's list");
+        return row_lin<at % 16>(sys.tab[at / 16], v...);
+    } else {
+        return (... + (tab_entry<K>(sys, ofs) * v));
+    }
+}
+// acc + and acc - the entries K... times v..., in order
+template <class Sys, int... K, class... V>
+__device__ __forceinline__ double lin_add(const Sys &sys, int ofs, Entries<K...> e, double acc,
+                                          V... v) {
+    if constexpr (row_tableau<Sys>::value) {
+        constexpr int at = row_slot(Entries<K...>{});
+        static_assert(at >= 0, "not in the row's list");
+        return row_add<at % 16>(sys.tab[at / 16], acc, v...);
+    } else {
+        return (acc + ... + (tab_entry<K>(sys, ofs) * v));
+    }
+}
+template <class Sys, int... K, class... V>
+__device__ __forceinline__ double lin_sub(const Sys &sys, int ofs, Entries<K...> e, double acc,
+                                          V... v) {
+    if constexpr (row_tableau<Sys>::value)
+        return lin_add(sys, ofs, e, acc, v...);  // the row's list holds them negated
+    else
+        return (acc - ... - (tab_entry<K>(sys, ofs) * v));
 }
 
 // One step attempt (dopcor basic step, dop853.cpp:339-648) for the lane's NC
@@ -878,11 +1158,6 @@ __device__ __forceinline__ int dop_attempt(const DevPot &P, const DopArgs &a, co
     // registers and spill)
     int tofs = 0;
     if constexpr (lds_tableau<Sys>::value) asm volatile("" : "+v"(tofs));
-#define TAB_A(i, j) tab_entry(sys, tofs, TAB_OFS_A + (i) * 16 + (j), T::A[i][j])
-#define TAB_D(i, j) tab_entry(sys, tofs, TAB_OFS_D + (i) * 16 + (j), T::D[i][j])
-#define TAB_B(k) tab_entry(sys, tofs, TAB_OFS_B + (k), T::B[k])
-#define TAB_E5(k) tab_entry(sys, tofs, TAB_OFS_E5 + (k), T::E5[k])
-#define TAB_BHH(k) tab_entry(sys, tofs, TAB_OFS_BHH + (k), T::BHH[k])
     const double safe = 0.9, facc1 = 1.0 / 0.333, facc2 = 1.0 / 6.0;  // expo1 = 1/8
     if (s.nstep > a.nmax) return -2;
     if (0.1 * fabs(s.h) <= fabs(s.x) * a.uround) return -3;
@@ -891,42 +1166,38 @@ __device__ __forceinline__ int dop_attempt(const DevPot &P, const DopArgs &a, co
     s.h = h;
     s.nstep++;
     double k2[NC], k3[NC], k4[NC], k5[NC], k6[NC], k7[NC], k8[NC], k9[NC], k10[NC], yy[NC];
-    FORN yy[c] = y[c] + h * TAB_A(1, 0) * k1[c];
+    FORN yy[c] = y[c] + h * tab_entry<TAB_OFS_A + 16>(sys, tofs) * k1[c];
     sys.rhs(P, yy, k2);
-    FORN yy[c] = y[c] + h * (TAB_A(2, 0) * k1[c] + TAB_A(2, 1) * k2[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<2, 0, 1>{}, k1[c], k2[c]);
     sys.rhs(P, yy, k3);
-    FORN yy[c] = y[c] + h * (TAB_A(3, 0) * k1[c] + TAB_A(3, 2) * k3[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<3, 0, 2>{}, k1[c], k3[c]);
     sys.rhs(P, yy, k4);
-    FORN yy[c] = y[c] + h * (TAB_A(4, 0) * k1[c] + TAB_A(4, 2) * k3[c] + TAB_A(4, 3) * k4[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<4, 0, 2, 3>{}, k1[c], k3[c], k4[c]);
     sys.rhs(P, yy, k5);
-    FORN yy[c] = y[c] + h * (TAB_A(5, 0) * k1[c] + TAB_A(5, 3) * k4[c] + TAB_A(5, 4) * k5[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<5, 0, 3, 4>{}, k1[c], k4[c], k5[c]);
     sys.rhs(P, yy, k6);
-    FORN yy[c] = y[c] + h * (TAB_A(6, 0) * k1[c] + TAB_A(6, 3) * k4[c] + TAB_A(6, 4) * k5[c] +
-                             TAB_A(6, 5) * k6[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<6, 0, 3, 4, 5>{}, k1[c], k4[c], k5[c], k6[c]);
     sys.rhs(P, yy, k7);
-    FORN yy[c] = y[c] + h * (TAB_A(7, 0) * k1[c] + TAB_A(7, 3) * k4[c] + TAB_A(7, 4) * k5[c] +
-                             TAB_A(7, 5) * k6[c] + TAB_A(7, 6) * k7[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<7, 0, 3, 4, 5, 6>{}, k1[c], k4[c], k5[c],
+                                k6[c], k7[c]);
     sys.rhs(P, yy, k8);
-    FORN yy[c] = y[c] + h * (TAB_A(8, 0) * k1[c] + TAB_A(8, 3) * k4[c] + TAB_A(8, 4) * k5[c] +
-                             TAB_A(8, 5) * k6[c] + TAB_A(8, 6) * k7[c] + TAB_A(8, 7) * k8[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<8, 0, 3, 4, 5, 6, 7>{}, k1[c], k4[c], k5[c],
+                                k6[c], k7[c], k8[c]);
     sys.rhs(P, yy, k9);
-    FORN yy[c] = y[c] + h * (TAB_A(9, 0) * k1[c] + TAB_A(9, 3) * k4[c] + TAB_A(9, 4) * k5[c] +
-                             TAB_A(9, 5) * k6[c] + TAB_A(9, 6) * k7[c] + TAB_A(9, 7) * k8[c] +
-                             TAB_A(9, 8) * k9[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<9, 0, 3, 4, 5, 6, 7, 8>{}, k1[c], k4[c],
+                                k5[c], k6[c], k7[c], k8[c], k9[c]);
     sys.rhs(P, yy, k10);
-    FORN yy[c] = y[c] + h * (TAB_A(10, 0) * k1[c] + TAB_A(10, 3) * k4[c] + TAB_A(10, 4) * k5[c] +
-                             TAB_A(10, 5) * k6[c] + TAB_A(10, 6) * k7[c] + TAB_A(10, 7) * k8[c] +
-                             TAB_A(10, 8) * k9[c] + TAB_A(10, 9) * k10[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<10, 0, 3, 4, 5, 6, 7, 8, 9>{}, k1[c], k4[c],
+                                k5[c], k6[c], k7[c], k8[c], k9[c], k10[c]);
     sys.rhs(P, yy, k2);  // stage 11 reuses k2 (dop853.cpp:402)
     const double xph = s.x + h;
-    FORN yy[c] = y[c] + h * (TAB_A(11, 0) * k1[c] + TAB_A(11, 3) * k4[c] + TAB_A(11, 4) * k5[c] +
-                             TAB_A(11, 5) * k6[c] + TAB_A(11, 6) * k7[c] + TAB_A(11, 7) * k8[c] +
-                             TAB_A(11, 8) * k9[c] + TAB_A(11, 9) * k10[c] + TAB_A(11, 10) * k2[c]);
+    FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<11, 0, 3, 4, 5, 6, 7, 8, 9, 10>{}, k1[c],
+                                k4[c], k5[c], k6[c], k7[c], k8[c], k9[c], k10[c], k2[c]);
     sys.rhs(P, yy, k3);  // stage 12 reuses k3 (:408)
     s.nfcn += 11;
     FORN {
-        k4[c] = TAB_B(0) * k1[c] + TAB_B(5) * k6[c] + TAB_B(6) * k7[c] + TAB_B(7) * k8[c] +
-                TAB_B(8) * k9[c] + TAB_B(9) * k10[c] + TAB_B(10) * k2[c] + TAB_B(11) * k3[c];
+        k4[c] = lin(sys, tofs, EntriesB<0, 5, 6, 7, 8, 9, 10, 11>{}, k1[c], k6[c], k7[c], k8[c],
+                    k9[c], k10[c], k2[c], k3[c]);
         k5[c] = y[c] + h * k4[c];
     }
     // error estimation (:416-444), n = 6; one divide serves both estimates
@@ -934,10 +1205,10 @@ __device__ __forceinline__ int dop_attempt(const DevPot &P, const DopArgs &a, co
     FORN {
         const double sk = a.atol + a.rtol * max_d(fabs(y[c]), fabs(k5[c]));
         const double isk = 1.0 / sk;
-        double erri = k4[c] - TAB_BHH(0) * k1[c] - TAB_BHH(8) * k9[c] - TAB_BHH(11) * k3[c];
+        double erri = lin_sub(sys, tofs, EntriesBHH<0, 8, 11>{}, k4[c], k1[c], k9[c], k3[c]);
         e2[c] = erri * isk;
-        erri = TAB_E5(0) * k1[c] + TAB_E5(5) * k6[c] + TAB_E5(6) * k7[c] + TAB_E5(7) * k8[c] +
-               TAB_E5(8) * k9[c] + TAB_E5(9) * k10[c] + TAB_E5(10) * k2[c] + TAB_E5(11) * k3[c];
+        erri = lin(sys, tofs, EntriesE5<0, 5, 6, 7, 8, 9, 10, 11>{}, k1[c], k6[c], k7[c], k8[c],
+                   k9[c], k10[c], k2[c], k3[c]);
         e1[c] = erri * isk;
     }
     double err = 0.0, err2 = 0.0;
@@ -988,44 +1259,34 @@ __device__ __forceinline__ int dop_attempt(const DevPot &P, const DopArgs &a, co
                     const double bspl = h * k1[c] - ydiff;
                     r3[c] = bspl;
                     r4[c] = ydiff - h * k4[c] - bspl;
-                    r5[c] = TAB_D(0, 0) * k1[c] + TAB_D(0, 5) * k6[c] + TAB_D(0, 6) * k7[c] +
-                            TAB_D(0, 7) * k8[c] + TAB_D(0, 8) * k9[c] + TAB_D(0, 9) * k10[c] +
-                            TAB_D(0, 10) * k2[c] + TAB_D(0, 11) * k3[c];
-                    r6[c] = TAB_D(1, 0) * k1[c] + TAB_D(1, 5) * k6[c] + TAB_D(1, 6) * k7[c] +
-                            TAB_D(1, 7) * k8[c] + TAB_D(1, 8) * k9[c] + TAB_D(1, 9) * k10[c] +
-                            TAB_D(1, 10) * k2[c] + TAB_D(1, 11) * k3[c];
-                    r7[c] = TAB_D(2, 0) * k1[c] + TAB_D(2, 5) * k6[c] + TAB_D(2, 6) * k7[c] +
-                            TAB_D(2, 7) * k8[c] + TAB_D(2, 8) * k9[c] + TAB_D(2, 9) * k10[c] +
-                            TAB_D(2, 10) * k2[c] + TAB_D(2, 11) * k3[c];
-                    r8[c] = TAB_D(3, 0) * k1[c] + TAB_D(3, 5) * k6[c] + TAB_D(3, 6) * k7[c] +
-                            TAB_D(3, 7) * k8[c] + TAB_D(3, 8) * k9[c] + TAB_D(3, 9) * k10[c] +
-                            TAB_D(3, 10) * k2[c] + TAB_D(3, 11) * k3[c];
+                    r5[c] = lin(sys, tofs, EntriesD<0, 0, 5, 6, 7, 8, 9, 10, 11>{}, k1[c], k6[c],
+                                k7[c], k8[c], k9[c], k10[c], k2[c], k3[c]);
+                    r6[c] = lin(sys, tofs, EntriesD<1, 0, 5, 6, 7, 8, 9, 10, 11>{}, k1[c], k6[c],
+                                k7[c], k8[c], k9[c], k10[c], k2[c], k3[c]);
+                    r7[c] = lin(sys, tofs, EntriesD<2, 0, 5, 6, 7, 8, 9, 10, 11>{}, k1[c], k6[c],
+                                k7[c], k8[c], k9[c], k10[c], k2[c], k3[c]);
+                    r8[c] = lin(sys, tofs, EntriesD<3, 0, 5, 6, 7, 8, 9, 10, 11>{}, k1[c], k6[c],
+                                k7[c], k8[c], k9[c], k10[c], k2[c], k3[c]);
                 }
-                FORN yy[c] = y[c] + h * (TAB_A(13, 0) * k1[c] + TAB_A(13, 6) * k7[c] +
-                                         TAB_A(13, 7) * k8[c] + TAB_A(13, 8) * k9[c] +
-                                         TAB_A(13, 9) * k10[c] + TAB_A(13, 10) * k2[c] +
-                                         TAB_A(13, 11) * k3[c] + TAB_A(13, 12) * k4[c]);
+                FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<13, 0, 6, 7, 8, 9, 10, 11, 12>{},
+                                            k1[c], k7[c], k8[c], k9[c], k10[c], k2[c], k3[c], k4[c]);
                 sys.rhs(P, yy, k10);
-                FORN yy[c] = y[c] + h * (TAB_A(14, 0) * k1[c] + TAB_A(14, 5) * k6[c] +
-                                         TAB_A(14, 6) * k7[c] + TAB_A(14, 7) * k8[c] +
-                                         TAB_A(14, 10) * k2[c] + TAB_A(14, 11) * k3[c] +
-                                         TAB_A(14, 12) * k4[c] + TAB_A(14, 13) * k10[c]);
+                FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<14, 0, 5, 6, 7, 10, 11, 12, 13>{},
+                                            k1[c], k6[c], k7[c], k8[c], k2[c], k3[c], k4[c], k10[c]);
                 sys.rhs(P, yy, k2);
-                FORN yy[c] = y[c] + h * (TAB_A(15, 0) * k1[c] + TAB_A(15, 5) * k6[c] +
-                                         TAB_A(15, 6) * k7[c] + TAB_A(15, 7) * k8[c] +
-                                         TAB_A(15, 8) * k9[c] + TAB_A(15, 12) * k4[c] +
-                                         TAB_A(15, 13) * k10[c] + TAB_A(15, 14) * k2[c]);
+                FORN yy[c] = y[c] + h * lin(sys, tofs, EntriesA<15, 0, 5, 6, 7, 8, 12, 13, 14>{},
+                                            k1[c], k6[c], k7[c], k8[c], k9[c], k4[c], k10[c], k2[c]);
                 sys.rhs(P, yy, k3);
                 s.nfcn += 3;
                 FORN {
-                    r5[c] = h * (r5[c] + TAB_D(0, 12) * k4[c] + TAB_D(0, 13) * k10[c] +
-                                 TAB_D(0, 14) * k2[c] + TAB_D(0, 15) * k3[c]);
-                    r6[c] = h * (r6[c] + TAB_D(1, 12) * k4[c] + TAB_D(1, 13) * k10[c] +
-                                 TAB_D(1, 14) * k2[c] + TAB_D(1, 15) * k3[c]);
-                    r7[c] = h * (r7[c] + TAB_D(2, 12) * k4[c] + TAB_D(2, 13) * k10[c] +
-                                 TAB_D(2, 14) * k2[c] + TAB_D(2, 15) * k3[c]);
-                    r8[c] = h * (r8[c] + TAB_D(3, 12) * k4[c] + TAB_D(3, 13) * k10[c] +
-                                 TAB_D(3, 14) * k2[c] + TAB_D(3, 15) * k3[c]);
+                    r5[c] = h * lin_add(sys, tofs, EntriesD<0, 12, 13, 14, 15>{}, r5[c], k4[c],
+                                        k10[c], k2[c], k3[c]);
+                    r6[c] = h * lin_add(sys, tofs, EntriesD<1, 12, 13, 14, 15>{}, r6[c], k4[c],
+                                        k10[c], k2[c], k3[c]);
+                    r7[c] = h * lin_add(sys, tofs, EntriesD<2, 12, 13, 14, 15>{}, r7[c], k4[c],
+                                        k10[c], k2[c], k3[c]);
+                    r8[c] = h * lin_add(sys, tofs, EntriesD<3, 12, 13, 14, 15>{}, r8[c], k4[c],
+                                        k10[c], k2[c], k3[c]);
                 }
                 const double x0 = s.x, x1 = s.x + h;
                 while (s.oidx < a.out_end) {
@@ -1070,11 +1331,6 @@ __device__ __forceinline__ int dop_attempt(const DevPot &P, const DopArgs &a, co
     }
     if (code == 0) s.h = hnew;
     return code;
-#undef TAB_A
-#undef TAB_D
-#undef TAB_B
-#undef TAB_E5
-#undef TAB_BHH
 }
 
 __device__ __forceinline__ void finish_stats(const DopArgs &a, const DopState &s, int code) {
@@ -1125,7 +1381,7 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
                                        const double (&k16)[6]) {
     const int lane = threadIdx.x & 63;
     const int row = lane / WIDE_ROW, c = lane % WIDE_ROW;
-    const int comp = c < 12 ? c % 6 : (c - 9 < 5 ? c - 9 : 5);
+    const WideRow<SCF, LAY, DENSE> row_sys(P, c);
     unsigned long long m = __ballot(active);
     for (int i = 0; i < row; i++) m &= m - 1ull;  // the row-th active lane
     bool ract = m != 0ull;
@@ -1134,7 +1390,7 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
 #pragma unroll
     for (int j = 0; j < 6; j++) {
         const double vy = from_lane(y6[j], src), vk = from_lane(k16[j], src);
-        if (comp == j) {
+        if (row_sys.comp == j) {
             y[0] = vy;
             k1[0] = vk;
         }
@@ -1158,13 +1414,12 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
     s.iasti = from_lane(s6.iasti, src);
     s.nonsti = from_lane(s6.nonsti, src);
     s.pend = 0;
-    const WideRow<SCF, LAY> row_sys{comp, c < 6};
     // every row ends: each attempt advances nstep, and nmax bounds it
     while (__any(ract)) {
         if (ract) {
             const int code = dop_attempt<SCF, DENSE, LAY>(P, a, row_sys, s, y, k1);
             if (code != 0) {
-                if (c < 6) a.w_final[c * a.N + s.orb] = y[0];
+                if (row_sys.writes) a.w_final[row_sys.comp * a.N + s.orb] = y[0];
                 if (c == 0) finish_stats(a, s, code);
                 ract = false;
             }

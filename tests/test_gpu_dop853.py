@@ -177,6 +177,52 @@ def test_wide_tail_matches_one_lane_per_orbit(layout, monkeypatch):
     assert np.all(out["2", 0][1] == 1)
 
 
+@pytest.mark.parametrize("n", [1, 4, 5, 17, 65])
+def test_rows_equal_one_lane_on_extreme_orbits(n, monkeypatch):
+    """A row's lanes hold one component each, take the tableau from each
+    other's registers and share the Milky-Way evaluator's roots and logarithm;
+    whatever the state, the results are one lane's, bit for bit: planar orbits
+    (zeros of either sign), orbits through the centre, radii where the shared
+    reciprocal over- or underflows, a start at the centre (NaN), with and
+    without dense output, for a few steps at least."""
+    from gala_amd.integrate import dop853
+    from gala_amd import _device as dev
+    rng = np.random.default_rng(31)
+    w0 = np.vstack([rng.uniform(-20, 20, (3, n)), rng.normal(0, 0.12, (3, n))])
+    edge = np.zeros((6, 9))
+    edge[:, 0] = [8.0, 0.0, 0.0, 0.0, 0.2, 0.0]
+    edge[:, 1] = [8.0, -0.0, -0.0, 0.0, -0.2, -0.0]
+    edge[:, 2] = [0.0, 0.0, 5.0, 0.0, 0.0, 0.1]
+    edge[:, 3] = [1e-3, 0.0, 0.0, 0.0, 1e-3, 0.0]
+    edge[:, 4] = [1e100, 1e99, -1e100, 0.1, 0.2, 0.3]
+    edge[:, 5] = [1e-100, 1e-101, 1e-100, 0.0, 0.0, 1e-5]
+    edge[:, 6] = [0.0, 0.0, 0.0, 0.1, 0.0, 0.0]
+    edge[:, 7] = [3.0, 1e-310, 2.0, -0.1, 0.0, 1e-310]
+    edge[:, 8] = [1e160, 0.0, 0.0, 0.0, 0.0, 0.0]
+    m = min(n, 9)
+    w0[:, n - m:] = edge[:, 9 - m:]
+    pot = mw_product()
+    t_out = np.linspace(0.0, 40.0, 9)
+    out = {}
+    for wide in ("0", "1", "2"):
+        monkeypatch.setenv("GAMD_DOP853_WIDE", wide)
+        for dense in (None, t_out):
+            r = dop853(pot, w0, 0.0, 40.0, 1.0, rtol=1e-8, atol=1e-10, nmax=300, t_out=dense,
+                       n_tail=n)
+            out[wide, dense is None] = [dev.to_host(r[k]) for k in ("w_final", "status", "stats")]
+            if dense is not None:
+                done = out[wide, False][1] == 1
+                out[wide, False].append(dev.to_host(r["w_out"])[:, :, done])
+    for wide in ("1", "2"):
+        for final_only in (True, False):
+            for a, b in zip(out["0", final_only], out[wide, final_only]):
+                same = a == b
+                if a.dtype == np.float64:  # NaN equals NaN; zeros keep their sign
+                    same = np.where(np.isnan(a), np.isnan(b),
+                                    same & (np.signbit(a) == np.signbit(b)))
+                assert np.all(same), (wide, final_only)
+
+
 def test_dedicated_tail_waves_match():
     """n_tail > 0 runs the queue order's first orbits on dedicated 16-lane
     rows from the start; the results are those of the one-lane kernel, bit
