@@ -32,6 +32,7 @@
 
 #include "dop853_tableau.h"
 #include "gamd_host.hpp"
+#include "gamd_row.hpp"
 
 using namespace gamd;
 namespace T = gamd::dop;
@@ -139,17 +140,6 @@ __device__ double hinit(const DevPot &P, double x, const double *y, double posne
 constexpr int WIDE_ROW = 16;   // lanes per orbit in the wide tail (one DPP row)
 constexpr int WIDE_ORBITS = 4; // orbits per wave in the wide tail
 constexpr int QUAD_ORBITS = 16; // orbits per wave in the quad tail (one per 4-lane quad)
-
-// llvm.amdgcn.update.dpp on a double: one v_mov_b64_dpp (the builtin takes 32 bits)
-__device__ double dpp_f64(double old, double v, int ctrl, int row_mask, int bank_mask,
-                          bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.f64");
-
-template <int SRC>
-__device__ __forceinline__ double row_bcast(double v) {
-    // DPP row_newbcast:SRC: every lane of a 16-lane row reads lane SRC of the
-    // row (every lane has a source in its row, so the zero is not used)
-    return dpp_f64(0.0, v, 0x150 + SRC, 0xF, 0xF, true);
-}
 
 // DPP row_half_mirror: lane i of 8 reads lane 7 - i
 __device__ __forceinline__ double half_mirror(double v) {
@@ -515,45 +505,6 @@ __device__ __forceinline__ double row_add(double t, double acc, V... v) {
 #undef GAMD_TERMS9
 #undef GAMD_LANES
 
-// The Milky-Way evaluator (mw_factors) on a 16-lane row whose lanes 0 to 7
-// use its result: the two reciprocal roots that do not wait for each other are
-// one, of r^2 in the lower and of z^2 + b^2 in the upper half, and the log's
-// polynomial is one chain of three lanes' coefficients instead of three.  The
-// same operations on the same values; a wave alone on its SIMD waits for the
-// issue of every instruction, of which an evaluation loses 8 in 117.
-struct RowMw {
-    MwConstants m;
-    double lo0, lo1, hi0, hi1;  // lane i: the i-th third of log_poly's coefficients
-    bool upper;
-    __device__ __forceinline__ RowMw(const DevPot &P, int lane) : m(P), upper(lane >= 8) {
-        lo0 = lane == 0 ? 1.0 : (lane == 1 ? 0.1111111111111111 : 0.058823529411764705);
-        lo1 = lane == 0 ? 0.3333333333333333
-                        : (lane == 1 ? 0.09090909090909091 : 0.05263157894736842);
-        hi0 = lane == 0 ? 0.2 : (lane == 1 ? 0.07692307692307693 : 0.047619047619047616);
-        hi1 = lane == 0 ? 0.14285714285714285
-                        : (lane == 1 ? 0.06666666666666667 : 0.043478260869565216);
-        // kept in vector registers: as scalars they were read again from
-        // memory, with a wait each, in every attempt
-        asm volatile("" : "+v"(m.m1), "+v"(m.c1), "+v"(m.m2), "+v"(m.c2), "+v"(m.m3), "+v"(m.a3),
-                     "+v"(m.b3sq), "+v"(m.m4), "+v"(m.irs4));
-        asm volatile("" : "+v"(lo0), "+v"(lo1), "+v"(hi0), "+v"(hi1));
-    }
-    __device__ __forceinline__ void rsqrt_pair(double a, double b, double &ra, double &rb) const {
-        ra = rsqrt_nr(upper ? b : a);
-        rb = row_bcast<8>(ra);
-    }
-    __device__ __forceinline__ double operator()(double z, double z2, double z4, double z8) const {
-        const double q = fma(z2, fma(z, hi1, hi0), fma(z, lo1, lo0));
-        double r;
-        asm("s_nop 1\n"
-            "v_mov_b64_dpp %0, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-            "v_fmac_f64_dpp %0, %1, %3 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-            : "=&v"(r)
-            : "v"(q), "v"(z4), "v"(z8));
-        return r;
-    }
-};
 struct NoRowMw {
     __device__ __forceinline__ NoRowMw(const DevPot &, int) {}
 };

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "gamd_host.hpp"
+#include "gamd_row.hpp"
 
 using namespace gamd;
 
@@ -44,7 +45,8 @@ __global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_leapfrog(con
     if (i >= N) return;
     double x = w0[i], y = w0[N + i], z = w0[2 * N + i];
     double vx = w0[3 * N + i], vy = w0[4 * N + i], vz = w0[5 * N + i];
-    const int64_t ns = nsteps_i ? nsteps_i[i] : n_steps;
+    // saved grids have one length: a scalar loop count
+    const int64_t ns = !SAVE && nsteps_i ? nsteps_i[i] : n_steps;
     if (SAVE) {
         const int64_t s = (int64_t)nsave * N;
         wout[i] = x;
@@ -176,6 +178,15 @@ auto by_layout(const gamd_potential *pot, F f) {
 }
 
 constexpr unsigned LF_BLOCK = 64;  // one wave per workgroup spreads small N over all CUs
+// Rows: a workgroup's 16 orbits are one 128-byte line of every saved row.
+constexpr unsigned LF_ROW = 16, LF_ROW_BLOCK = 256;
+// k_leapfrog_row while every row's wave has a SIMD for itself (two to a SIMD take
+// twice as long), ns per step on rows and one orbit a lane: every step saved, 16 to
+// 1,024 orbits 266-270 and 322, 4,096 orbits 300 and 323; final states only, 229-231
+// and 256, 2,048 orbits 241 and 256, 4,096 orbits 264 and 256.
+inline bool lf_rows(int layout, size_t N, int64_t n_steps, bool saved) {
+    return layout == LAYOUT_MW && N <= (saved ? 4096 : 2048) && n_steps < INT32_MAX;
+}
 
 // ---------------------------------------------------------------------------
 // Streamed saved trajectory: one chunk of `rows` saved rows [row0, row0 +
@@ -279,6 +290,87 @@ __global__ __launch_bounds__(SCF ? 64 : 256, scf_waves(LAY)) void k_leapfrog_chu
     }
 }
 
+// The same integration of a few orbits in the Milky-Way layout, one orbit per
+// 16-lane row: lanes c and 8 + c hold the position and velocity along axis
+// min(c, 2), take the others by row broadcasts and need the gradient along their
+// own axis only.  All lanes of an axis hold and store the same values: a mask
+// around the stores costs a lone wave more.  Same operations on the same values as one lane per
+// orbit.  A wave alone on its SIMD pays the issue of every instruction of a
+// step, ~4 cycles each whatever it does: one orbit a lane 115 for the force and
+// the kick and some 20 for the loop, here 103 and 8.
+// slot = nullptr: nothing is saved (rows = 1); w_final may be nullptr.  Counts
+// are 32 bits: a 64-bit counter and its compare are scalar instructions that the
+// wave waits for like any other.
+__global__ __launch_bounds__(LF_ROW_BLOCK) void k_leapfrog_row(const DevPot *__restrict__ Pp,
+                                                               ChunkArgs a) {
+    const DevPot &P = *Pp;
+    const int64_t i = (blockIdx.x * (int64_t)LF_ROW_BLOCK + threadIdx.x) / LF_ROW;
+    if (i >= a.N) return;  // whole rows
+    const int lane = threadIdx.x % LF_ROW;
+    const int axis = (lane & 7) < 3 ? (lane & 7) : 2;
+    const RowMwAll mw(P, lane);
+    const int64_t N = a.N, so = a.rows_max * N;
+    const double dt = a.dt;
+    const int64_t at = axis * N + i;
+    auto grad = [&](double q) {
+        return mw_grad_along(P, mw.m, mw, row_bcast<0>(q), row_bcast<1>(q), row_bcast<2>(q), axis,
+                             q);
+    };
+    double q, v, h, g = 0.0;
+    double *qo = a.slot + axis * so + i, *vo = qo + 3 * so;  // the next saved row's entries
+    double from = 0.0;
+    auto step = [&] {
+        q = q + h * dt;
+        g = grad(q);
+        from = h;
+        h = h - g * dt;
+    };
+    uint32_t rows = (uint32_t)a.rows;
+    if (a.first) {
+        q = a.w0[at];
+        v = a.w0[3 * N + at];
+        if (a.slot) {
+            *qo = q;
+            *vo = v;
+            qo += N;
+            vo += N;
+        }
+        rows--;
+        h = v - grad(q) * dt / 2.0;
+    } else {
+        q = a.state[at];
+        h = a.state[3 * N + at];
+        v = h;
+    }
+    const uint32_t between = (uint32_t)a.stride - 1;
+    for (; rows; rows--) {
+        for (uint32_t k = between; k; k--) step();
+        step();
+        v = fma(-0.5, g * dt, from);
+        *qo = q;
+        *vo = v;
+        qo += N;
+        vo += N;
+    }
+    // the last chunk goes on to n_steps
+    uint32_t tail = a.last ? (uint32_t)(a.n_steps - (a.row0 + a.rows - 1) * a.stride) : 0;
+    if (tail) {
+        do step();
+        while (--tail);
+        v = fma(-0.5, g * dt, from);
+    }
+    double *end = a.last ? a.w_final : a.state;
+    if (end) {
+        end[at] = q;
+        end[3 * N + at] = a.last ? v : h;
+    }
+}
+
+void launch_rows(const DevPot *P, const ChunkArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(k_leapfrog_row, dim3(grid_for((size_t)a.N * LF_ROW, LF_ROW_BLOCK)),
+                       dim3(LF_ROW_BLOCK), 0, s, P, a);
+}
+
 // The chunk sequence on the compute stream s, with each chunk's rows copied
 // to the host on stream c while the next chunk computes (two ring slots; a
 // slot is rewritten only after its copy has finished).  Both streams end
@@ -309,7 +401,10 @@ int stream_chunks(const DevPot *P, const double *w0, size_t N, double dt, int64_
         a.dt = dt;
         a.first = k == 0;
         a.last = k == nchunk - 1;
-        hipLaunchKernelGGL((k_leapfrog_chunk<SCF, LAY>), dim3(g), dim3(LF_BLOCK), 0, s, P, a);
+        if (lf_rows(LAY, N, n_steps, true))
+            launch_rows(P, a, s);
+        else
+            hipLaunchKernelGGL((k_leapfrog_chunk<SCF, LAY>), dim3(g), dim3(LF_BLOCK), 0, s, P, a);
         const int rc = launch_status();
         if (rc != GAMD_OK) return rc;
         GAMD_HIP_CHECK(hipEventRecord(comp, s));
@@ -339,6 +434,20 @@ extern "C" int gamd_leapfrog(const gamd_potential *pot, const double *w0, size_t
     const int64_t nsave = w_out ? n_steps / save_stride + 1 : 0;
     const unsigned g = grid_for(N, LF_BLOCK);
     hipStream_t s = as_stream(stream);
+    if (lf_rows(pot->dev.layout, N, n_steps, w_out != nullptr) && !n_steps_per_orbit) {
+        ChunkArgs a = {};
+        a.w0 = w0;
+        a.slot = w_out;
+        a.w_final = w_final;
+        a.N = (int64_t)N;
+        a.rows = a.rows_max = w_out ? nsave : 1;
+        a.stride = w_out ? save_stride : 1;
+        a.n_steps = n_steps;
+        a.dt = dt;
+        a.first = a.last = 1;
+        launch_rows(pot->ddev, a, s);
+        return launch_status();
+    }
     auto kern = by_layout(pot, [&](auto scf, auto lay) {
         return w_out ? k_leapfrog<scf.value, true, lay.value> : k_leapfrog<scf.value, false, lay.value>;
     });
@@ -371,7 +480,6 @@ extern "C" int gamd_leapfrog_stream(const gamd_potential *pot, const double *w0,
                                     int64_t chunk_rows, int use_graph, double *host_out,
                                     double *w_final, void *workspace, size_t workspace_bytes,
                                     void *stream) {
-    (void)t0;  // static potentials only
     if (!pot || !w0 || !host_out || !w_final || !workspace || n_steps < 0 || save_stride < 1 ||
         chunk_rows < 1)
         return GAMD_ERR_INVALID;
@@ -381,6 +489,19 @@ extern "C" int gamd_leapfrog_stream(const gamd_potential *pot, const double *w0,
     double *ring = static_cast<double *>(workspace);
     double *state = ring + 2 * 6 * (size_t)chunk_rows * N;
     hipStream_t s = as_stream(stream);
+    const int64_t nsave = n_steps / save_stride + 1;
+    if (chunk_rows >= nsave && !use_graph) {
+        // all rows in one chunk: nothing overlaps, so one kernel into the ring
+        // and one copy, without a second stream and its events (one orbit,
+        // 1,000 steps: the call 698 -> 393 us, with k_leapfrog_row)
+        const int rc = gamd_leapfrog(pot, w0, N, t0, dt, n_steps, nullptr, save_stride, ring,
+                                     w_final, stream);
+        if (rc != GAMD_OK) return rc;
+        GAMD_HIP_CHECK(hipMemcpyAsync(host_out, ring, 6 * (size_t)nsave * N * sizeof(double),
+                                      hipMemcpyDeviceToHost, s));
+        GAMD_HIP_CHECK(hipStreamSynchronize(s));
+        return GAMD_OK;
+    }
     hipStream_t c = nullptr, cs = nullptr;
     hipEvent_t comp = nullptr, copied[2] = {nullptr, nullptr};
     hipGraph_t graph = nullptr;

@@ -223,3 +223,28 @@ def test_milky_way_layout_at_extreme_radii(r):
     a, b = (dev.to_host(leapfrog(p, w0, 1e-3, 1, save=False)[1]) for p in (mw, general))
     np.testing.assert_allclose(a, b, rtol=4e-13, atol=0.0, equal_nan=True)
     assert np.isfinite(a[:, 1:40]).all()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 2048, 2049, 4096, 4097])
+@pytest.mark.parametrize("n_steps,stride", [(0, 1), (1, 1), (40, 1), (41, 3), (5, 8)])
+def test_few_orbits_on_rows_equal_one_orbit_a_lane(n, n_steps, stride):
+    """Up to 2,048 orbits of the Milky-Way layout (4,096 where rows are saved)
+    run one to a 16-lane row: saved rows and final states equal the same
+    orbits' in a launch of 4,200, one orbit a lane, bit for bit, and streamed
+    to the host in one chunk or several as well."""
+    from gala_amd import _device as dev
+    from gala_amd.integrate import leapfrog, leapfrog_to_host
+    pot = mw_product()
+    w0, dt, _ = workloads.composite_leapfrog(vcirc_oracle(mw_oracle()), n=4200, seed=9)
+    w0[:, n - 1] = [1e-145, 0.0, 0.0, 0.0, 0.0, 0.0]  # where the shared reciprocal gives way
+    ref, ref_fin = (dev.to_host(a)[..., :n] for a in leapfrog(pot, w0, dt, n_steps, stride))
+    few = np.ascontiguousarray(w0[:, :n])
+    out, fin = leapfrog(pot, few, dt, n_steps, stride)
+    np.testing.assert_array_equal(dev.to_host(out), ref)
+    np.testing.assert_array_equal(dev.to_host(fin), ref_fin)
+    np.testing.assert_array_equal(dev.to_host(leapfrog(pot, few, dt, n_steps, save=False)[1]),
+                                  ref_fin)
+    for rows in (4, ref.shape[1]):
+        out, fin = leapfrog_to_host(pot, few, dt, n_steps, stride, chunk_rows=rows)
+        np.testing.assert_array_equal(out, ref)
+        np.testing.assert_array_equal(dev.to_host(fin), ref_fin)
