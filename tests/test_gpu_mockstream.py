@@ -401,3 +401,42 @@ def test_one_body_lane_pairs_match_one_lane_kernel():
         one_lane = run([h, None], traj2)
         assert np.all(np.isfinite(pair))
         assert np.array_equal(pair, one_lane), h
+
+
+@pytest.mark.parametrize("body", ["plummer", "rotated plummer", "hernquist"])
+@pytest.mark.parametrize("n_steps", [0, 1, 2, 65])
+def test_one_body_pairs_equal_two_bodies(body, n_steps):
+    """The lane pairs' own straight line for one unrotated Plummer sphere, and
+    the component table for any other progenitor, equal the one-lane kernel
+    (selected by a second, massless body) bit for bit, from no step to more
+    steps than a wave has lanes, for a number of particles that fills no wave."""
+    from gala_amd import _device as dev
+    from gala_amd import _lib
+    from gala_amd.integrate import leapfrog
+    from gala_amd.potential import HernquistPotential, MilkyWayLikePotential, PlummerPotential
+    prog_w0, prog_mass, b, _, _ = workloads.mockstream_progenitor()
+    pot = {"plummer": lambda: PlummerPotential(m=prog_mass, b=b),
+           "rotated plummer": lambda: PlummerPotential(m=prog_mass, b=b,
+                                                       R=np.array([[0.0, 1, 0], [-1, 0, 0], [0, 0, 1]])),
+           "hernquist": lambda: HernquistPotential(m=prog_mass, c=b)}[body]()
+    ext, nfull, n = MilkyWayLikePotential(), n_steps + 1, 37
+    traj = dev.to_host(leapfrog(ext, prog_w0[:, None], 1.0, n_steps)[0])[:, :, 0]
+    rng = np.random.default_rng(11)
+    idx = np.arange(n) % nfull  # lengths differ within a wave
+    w0 = traj[:, idx] + np.vstack([rng.normal(0, 0.05, (3, n)), rng.normal(0, 0.002, (3, n))])
+    w0[:, 3] = traj[:, idx[3]]  # a particle at the progenitor's centre
+    w0d, reld, lib = dev.to_dev(w0), dev.to_dev(1.0 * idx), _lib.load()
+
+    def run(handles, tr):
+        out, trd = dev.empty((6, n)), dev.to_dev(np.ascontiguousarray(tr))
+        _lib.check(lib.gamd_mockstream_leapfrog(
+            ext.c_handle, _lib.body_array(handles), len(handles), trd.data_ptr(), nfull, 0.0, 1.0,
+            w0d.data_ptr(), reld.data_ptr(), n, float(n_steps), out.data_ptr(), dev.stream_ptr()),
+            "gamd_mockstream_leapfrog")
+        return dev.to_host(out)
+
+    two = run([pot.c_handle, None], np.stack([traj, traj + 40.0], axis=2))
+    centre = idx[3] == n_steps or body != "hernquist"  # Hernquist: 0/0 at its centre
+    keep = np.arange(n) != (n if centre else 3)
+    assert np.isfinite(two[:, keep]).all()
+    np.testing.assert_array_equal(run([pot.c_handle], traj), two)
