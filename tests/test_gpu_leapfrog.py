@@ -248,3 +248,34 @@ def test_few_orbits_on_rows_equal_one_orbit_a_lane(n, n_steps, stride):
         out, fin = leapfrog_to_host(pot, few, dt, n_steps, stride, chunk_rows=rows)
         np.testing.assert_array_equal(out, ref)
         np.testing.assert_array_equal(dev.to_host(fin), ref_fin)
+
+
+@pytest.mark.parametrize("n", [0, 1, 4097])
+def test_results_on_the_host_are_the_callers_own(n, monkeypatch):
+    """Host results (pinned up to a size and a total held) are separate, writable
+    arrays with the tensor's values, whichever memory they came back in, and
+    the total falls again when the last view of an array is gone."""
+    import gc
+    from gala_amd import _device as dev
+    t = dev.torch()
+    x = t.arange(6.0 * n, dtype=t.float64, device="cuda").reshape(6, n)
+    held = dev._pinned_held
+    a = dev.to_host(x)
+    assert dev._pinned_held == held + a.nbytes
+    monkeypatch.setattr(dev, "PINNED_HELD_BYTES", held + a.nbytes)
+    b = dev.to_host(x)  # no room (none needed where it is empty)
+    assert dev._pinned_held == held + a.nbytes
+    x.zero_()
+    want = np.arange(6.0 * n).reshape(6, n)
+    for got in (a, b, dev.to_host(t.from_numpy(want.T).cuda()).T):
+        np.testing.assert_array_equal(got, want)
+    a += 1.0
+    np.testing.assert_array_equal(b, want)
+    view = a[3:]
+    del a
+    gc.collect()
+    assert dev._pinned_held == held + 2 * view.nbytes
+    np.testing.assert_array_equal(view, want[3:] + 1.0)
+    del view, got
+    gc.collect()
+    assert dev._pinned_held == held
