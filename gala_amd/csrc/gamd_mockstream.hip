@@ -549,7 +549,7 @@ extern "C" int gamd_nbody_leapfrog(const gamd_potential *ext, const gamd_potenti
     if (n == 0) return GAMD_OK;
     // one body feels the external potential alone: gamd_leapfrog's arithmetic,
     // on its kernel for few orbits (4,000 steps of a stream's progenitor,
-    // every step saved: 2,017 -> 1,100 us)
+    // every step saved: 2,017 -> 1,060 us)
     if (n == 1)
         return gamd_leapfrog(ext, w0, 1, t0, dt, n_steps, nullptr, save_stride, w_out, w_final,
                              stream);
