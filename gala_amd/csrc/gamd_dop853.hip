@@ -1326,6 +1326,16 @@ __device__ __forceinline__ bool window_pause(const DopArgs &a, const WinArgs &w,
 // move to one 16-lane row each and are integrated to the end (or, in a
 // window of the dense output, to the window's end).  Called with every lane
 // of the wave converged; the queue is drained.
+// Up to FILL_ROWS_MAX orbits no lane is switched off before the last orbit ends: a
+// wave alone on its SIMD takes longer for the same instructions with part of its
+// lanes masked (a Leapfrog step of one row 258 ns, of four 228).  A row without
+// an orbit of its own, from the start or once that has ended, repeats another
+// row's and stores the same values.  One orbit 10.4 -> 9.2 ms, 1,500 uneven orbits
+// 51.0 -> 43.6, 8,000 83.1 -> 78.8.  Beyond that the rows' waves share their SIMDs, which
+// hides the loss, and full rows take issue slots from the others: 300,000 orbits
+// 93.3 and 93.1 ms, 1,048,576 87.4 and 88.6.
+constexpr int64_t FILL_ROWS_MAX = 65536;  // one wave of single lanes on each of 1,024 SIMDs
+
 template <bool SCF, bool DENSE, int LAY>
 __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, const WinArgs &w,
                                        bool active, const DopState &s6, const double (&y6)[6],
@@ -1333,10 +1343,11 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
     const int lane = threadIdx.x & 63;
     const int row = lane / WIDE_ROW, c = lane % WIDE_ROW;
     const WideRow<SCF, LAY, DENSE> row_sys(P, c);
-    unsigned long long m = __ballot(active);
+    const unsigned long long all = __ballot(active);
+    if (!all) return;
+    unsigned long long m = all;
     for (int i = 0; i < row; i++) m &= m - 1ull;  // the row-th active lane
-    bool ract = m != 0ull;
-    const int src = ract ? __ffsll((long long)m) - 1 : lane;
+    const int src = __ffsll((long long)(m ? m : all)) - 1;
     double y[1] = {0.0}, k1[1] = {0.0};
 #pragma unroll
     for (int j = 0; j < 6; j++) {
@@ -1366,7 +1377,9 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
     s.nonsti = from_lane(s6.nonsti, src);
     s.pend = 0;
     // every row ends: each attempt advances nstep, and nmax bounds it
-    while (__any(ract)) {
+    const bool fill = a.N <= FILL_ROWS_MAX;
+    bool ract = fill || m != 0ull;
+    while (true) {
         if (ract) {
             const int code = dop_attempt<SCF, DENSE, LAY>(P, a, row_sys, s, y, k1);
             if (code != 0) {
@@ -1376,6 +1389,31 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
             }
             if (window_pause<DENSE>(a, w, row_sys, s, y, k1, code)) ract = false;
         }
+        const unsigned long long live = __ballot(ract);
+        if (!live) break;
+        if (!fill || live == ~0ull) continue;
+        ract = true;
+        const int from = live >> lane & 1ull ? lane : __ffsll((long long)live) - 1 + c;
+        y[0] = from_lane(y[0], from);
+        k1[0] = from_lane(k1[0], from);
+        s.orb = from_lane(s.orb, from);
+        s.x = from_lane(s.x, from);
+        s.xend = from_lane(s.xend, from);
+        s.h = from_lane(s.h, from);
+        s.hmax = from_lane(s.hmax, from);
+        s.posneg = from_lane(s.posneg, from);
+        s.facold = from_lane(s.facold, from);
+        s.hlamb = from_lane(s.hlamb, from);
+        s.nstep = from_lane(s.nstep, from);
+        s.naccpt = from_lane(s.naccpt, from);
+        s.stiff = from_lane(s.stiff, from);
+        s.nrejct = from_lane(s.nrejct, from);
+        s.nfcn = from_lane(s.nfcn, from);
+        s.oidx = from_lane(s.oidx, from);
+        s.reject = from_lane(s.reject, from);
+        s.iasti = from_lane(s.iasti, from);
+        s.nonsti = from_lane(s.nonsti, from);
+        s.pend = from_lane(s.pend, from);
     }
 }
 

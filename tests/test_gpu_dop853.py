@@ -320,3 +320,30 @@ def test_order_entries_naming_no_orbit_are_skipped():
     assert np.array_equal(st[named], dev.to_host(ref["status"]))
     assert np.array_equal(dev.to_host(wfin)[:, named], dev.to_host(ref["w_final"]))
     assert np.array_equal(dev.to_host(stats)[named], dev.to_host(ref["stats"]))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 9])
+@pytest.mark.parametrize("nmax", [0, 40])
+def test_rows_without_an_orbit_repeat_another(n, nmax, monkeypatch):
+    """A few orbits of very different lengths, some stopped by nmax, on rows
+    from the start, from the queue's end or dedicated: a row whose orbit has
+    ended repeats another row's, and every orbit's final state, status, step
+    counts and dense samples are those of one lane per orbit, bit for bit."""
+    from gala_amd.integrate import dop853
+    from gala_amd import _device as dev
+    w0, _ = workloads.composite_dop853(vcirc_oracle(mw_oracle()), n=n, seed=5)
+    T = 40.0 * 3.0 ** (np.arange(n) % 4)
+    t_out = np.linspace(0.0, 40.0, 9)
+    out = {}
+    for wide, n_tail in (("0", 0), ("1", 0), ("2", 0), ("2", n)):
+        monkeypatch.setenv("GAMD_DOP853_WIDE", wide)
+        r = dop853(mw_product(), w0, 0.0, T, 1.0, rtol=1e-9, atol=1e-10, nmax=nmax, n_tail=n_tail)
+        d = dop853(mw_product(), w0, 0.0, T, 1.0, rtol=1e-9, atol=1e-10, nmax=nmax, n_tail=n_tail,
+                   t_out=t_out)
+        out[wide, n_tail] = [dev.to_host(r[k]) for k in ("w_final", "status", "stats")] + [
+            dev.to_host(d[k]) for k in ("w_final", "status", "stats")]
+        if not nmax:  # samples past an orbit's last step are left as they were
+            out[wide, n_tail].append(dev.to_host(d["w_out"]))
+    for got in out.values():
+        for a, b in zip(out["0", 0], got):
+            np.testing.assert_array_equal(a, b)
