@@ -279,3 +279,27 @@ def test_results_on_the_host_are_the_callers_own(n, monkeypatch):
     del view, got
     gc.collect()
     assert dev._pinned_held == held
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65])
+@pytest.mark.parametrize("name", ["composite", "nfw", "scf"])
+def test_partly_filled_waves_equal_full_ones(name, n):
+    """Lanes past the last orbit repeat it: the states and rows of a launch
+    whose last wave is not full are those of the same orbits in a larger one."""
+    from gala_amd import _device as dev
+    from gala_amd.integrate import leapfrog, ruth4
+    from gala_amd.potential import NFWPotential, SCFPotential
+    rng = np.random.default_rng(2)
+    if name == "scf":
+        S, T = workloads.scf_coefficients(3, 2, 1)
+        pot = SCFPotential(m=1e12, r_s=20.0, Snlm=S, Tnlm=T)
+    else:
+        pot = mw_product() if name == "composite" else NFWPotential(m=5.4e11, r_s=15.6)
+    w0 = np.vstack([rng.uniform(4.0, 20.0, (3, 4160)), rng.normal(0.0, 0.15, (3, 4160))])
+    few = np.ascontiguousarray(w0[:, :n])
+    for f in (leapfrog, ruth4):
+        for save in (True, False):
+            got, ref = f(pot, few, 1.0, 21, 4, save=save), f(pot, w0, 1.0, 21, 4, save=save)
+            for a, b in zip(got, ref):
+                if b is not None:
+                    np.testing.assert_array_equal(dev.to_host(a), dev.to_host(b)[..., :n])
