@@ -1,8 +1,5 @@
 """Device-memory plumbing: PyTorch-ROCm tensors hold the HBM buffers handed
 to the C ABI, and torch's current HIP stream orders the calls."""
-import threading
-import weakref
-
 import numpy as np
 
 
@@ -49,43 +46,8 @@ def ptr(x):
     return None if x is None else x.data_ptr()
 
 
-# Results come back in pinned memory (a copy into pageable memory goes through the
-# runtime's staging buffer and faults its pages in: 2.4 MB 149 us, pinned 51; 20 MB
-# 1,100 and 360) up to this size each and this much held by callers at a time:
-# pinned memory cannot be swapped out, and torch keeps its freed blocks for reuse.
-PINNED_RESULT_BYTES, PINNED_HELD_BYTES = 64 << 20, 1 << 30
-_pinned_held = 0
-_pinned_lock = threading.Lock()
-
-
-def _hold_pinned(nbytes):
-    global _pinned_held
-    with _pinned_lock:
-        if nbytes > 0 and _pinned_held + nbytes > PINNED_HELD_BYTES:
-            return False
-        _pinned_held += nbytes
-        return True
-
-
 def to_host(x):
-    """x as a numpy array in host memory"""
-    t = torch()
-    x = x.detach()
-    nbytes = x.numel() * x.element_size()
-    if (not x.is_cuda or not 0 < nbytes <= PINNED_RESULT_BYTES or not x.is_contiguous()
-            or not _hold_pinned(nbytes)):
-        return x.cpu().numpy()
-    try:
-        out = t.empty(x.shape, dtype=x.dtype, pin_memory=True)
-    except BaseException:
-        _hold_pinned(-nbytes)
-        raise
-    a = out.numpy()
-    # (a view's base is this array: it lives as long as any view does)
-    weakref.finalize(a, _hold_pinned, -nbytes).atexit = False
-    out.copy_(x, non_blocking=True)
-    t.cuda.current_stream(x.device).synchronize()
-    return a
+    return x.detach().cpu().numpy()
 
 
 def _shape(a):

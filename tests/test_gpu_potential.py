@@ -72,3 +72,38 @@ def test_nfw_special_cases():
     # gradient is 0/0 there (:844-845)
     assert p.energy(q)[0] == -p.G * 5.4e11 / 15.6
     assert np.all(np.isnan(p.gradient(q)))
+
+
+def _vm_flags(address):
+    """the kernel's flags of the mapping that holds address (/proc/self/smaps)"""
+    inside = False
+    with open("/proc/self/smaps") as f:
+        for line in f:
+            first = line.split()[0]
+            if not first.endswith(":"):
+                lo, hi = (int(v, 16) for v in first.split("-"))
+                inside = lo <= address < hi
+            elif inside and first == "VmFlags:":
+                return line.split()[1:]
+    raise AssertionError("no mapping holds the address")
+
+
+@pytest.mark.parametrize("n", [1, 4097, 400001])
+def test_results_can_be_read_in_a_forked_process(n):
+    """Results on the host lie in memory that a forked worker inherits (a data
+    loader's, a pool's), whatever their size: the driver's own pages do not go
+    through a fork ("dc") and reading them there ends the process."""
+    import os
+    q = _points(4, n=n)
+    results = [mw_product().energy(q), mw_product().gradient(q)]
+    want = [a.tobytes() for a in results]
+    for a in results:
+        for at in (a.ctypes.data, a.ctypes.data + a.nbytes - 1):
+            assert "dc" not in _vm_flags(at)
+    pid = os.fork()
+    if pid == 0:
+        try:
+            os._exit(0 if [a.tobytes() for a in results] == want else 1)
+        finally:
+            os._exit(2)
+    assert os.waitpid(pid, 0)[1] == 0
