@@ -33,6 +33,7 @@
 #include "dop853_tableau.h"
 #include "gamd_host.hpp"
 #include "gamd_row.hpp"
+#include "gamd_rules.hpp"
 
 using namespace gamd;
 namespace T = gamd::dop;
@@ -67,6 +68,7 @@ struct DopArgs {
     // windows)
     int64_t out_base, out_rows, out_end;
     double *pend;
+    bool fill_rows;        // wide_tail: rows without an orbit repeat another row's
 };
 
 #define FOR6 _Pragma("unroll") for (int c = 0; c < 6; c++)
@@ -1326,16 +1328,14 @@ __device__ __forceinline__ bool window_pause(const DopArgs &a, const WinArgs &w,
 // move to one 16-lane row each and are integrated to the end (or, in a
 // window of the dense output, to the window's end).  Called with every lane
 // of the wave converged; the queue is drained.
-// Up to FILL_ROWS_MAX orbits no lane is switched off before the last orbit ends: a
-// wave alone on its SIMD takes longer for the same instructions with part of its
-// lanes masked (a Leapfrog step of one row 258 ns, of four 228).  A row without
-// an orbit of its own, from the start or once that has ended, repeats another
-// row's and stores the same values.  One orbit 10.4 -> 9.2 ms, 1,500 uneven orbits
-// 51.0 -> 43.6, 8,000 83.1 -> 78.8.  Beyond that the rows' waves share their SIMDs, which
-// hides the loss, and full rows take issue slots from the others: 300,000 orbits
-// 93.3 and 93.1 ms, 1,048,576 87.4 and 88.6.
-constexpr int64_t FILL_ROWS_MAX = 65536;  // one wave of single lanes on each of 1,024 SIMDs
-
+// With a.fill_rows (up to filled_row_orbits() orbits, 65,536 on a whole chip) no
+// lane is switched off before the last orbit ends: a wave alone on its SIMD takes
+// longer for the same instructions with part of its lanes masked (a Leapfrog step of
+// one row 258 ns, of four 228).  A row without an orbit of its own, from the start or
+// once that has ended, repeats another row's and stores the same values.  One orbit
+// 10.4 -> 9.2 ms, 1,500 uneven orbits 51.0 -> 43.6, 8,000 83.1 -> 78.8.  Beyond that
+// the rows' waves share their SIMDs, which hides the loss, and full rows take issue
+// slots from the others: 300,000 orbits 93.3 and 93.1 ms, 1,048,576 87.4 and 88.6.
 template <bool SCF, bool DENSE, int LAY>
 __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, const WinArgs &w,
                                        bool active, const DopState &s6, const double (&y6)[6],
@@ -1377,7 +1377,7 @@ __device__ __forceinline__ void wide_tail(const DevPot &P, const DopArgs &a, con
     s.nonsti = from_lane(s6.nonsti, src);
     s.pend = 0;
     // every row ends: each attempt advances nstep, and nmax bounds it
-    const bool fill = a.N <= FILL_ROWS_MAX;
+    const bool fill = a.fill_rows;
     bool ract = fill || m != 0ull;
     while (true) {
         if (ract) {
@@ -2164,6 +2164,7 @@ DopArgs dop_args(const double *w0, size_t N, const double *t0, const double *t1,
     a.stats = stats;
     a.order = order;
     a.n_tail = n_tail;
+    a.fill_rows = a.N <= filled_row_orbits(cu_count());
     a.queue = queue;
     // GAMD_DOP853_WIDE=0 keeps one lane per orbit to the end, =1 skips the
     // quad stage (same results every way)

@@ -26,6 +26,7 @@
 
 #include "gamd_host.hpp"
 #include "gamd_row.hpp"
+#include "gamd_rules.hpp"
 
 using namespace gamd;
 
@@ -193,12 +194,9 @@ auto by_layout(const gamd_potential *pot, F f) {
 constexpr unsigned LF_BLOCK = 64;  // one wave per workgroup spreads small N over all CUs
 // Rows: a workgroup's 16 orbits are one 128-byte line of every saved row.
 constexpr unsigned LF_ROW = 16, LF_ROW_BLOCK = 256;
-// k_leapfrog_row while every row's wave has a SIMD for itself (two to a SIMD take
-// twice as long), ns per step on rows and one orbit a lane: every step saved, 16 to
-// 1,024 orbits 266-270 and 322, 4,096 orbits 300 and 323; final states only, 229-231
-// and 256, 2,048 orbits 241 and 256, 4,096 orbits 264 and 256.
 inline bool lf_rows(int layout, size_t N, int64_t n_steps, bool saved) {
-    return layout == LAYOUT_MW && N <= (saved ? 4096 : 2048) && n_steps < INT32_MAX;
+    return layout == LAYOUT_MW && n_steps < INT32_MAX &&
+           (int64_t)N <= leapfrog_row_orbits(cu_count(), saved);
 }
 
 // ---------------------------------------------------------------------------
@@ -390,11 +388,11 @@ void launch_rows(const DevPot *P, const ChunkArgs &a, hipStream_t s) {
 // The chunk sequence on the compute stream s, with each chunk's rows copied
 // to the host on stream c while the next chunk computes (two ring slots; a
 // slot is rewritten only after its copy has finished).  Both streams end
-// joined to s.
+// joined to s.  rows: one orbit to a 16-lane row.
 template <bool SCF, int LAY>
 int stream_chunks(const DevPot *P, const double *w0, size_t N, double dt, int64_t n_steps,
-                  int64_t stride, int64_t C, double *host_out, double *w_final, double *ring,
-                  double *state, hipStream_t s, hipStream_t c, hipEvent_t comp,
+                  int64_t stride, int64_t C, bool rows, double *host_out, double *w_final,
+                  double *ring, double *state, hipStream_t s, hipStream_t c, hipEvent_t comp,
                   hipEvent_t copied[2]) {
     const int64_t nsave = n_steps / stride + 1;
     const int64_t nchunk = (nsave + C - 1) / C;
@@ -417,7 +415,7 @@ int stream_chunks(const DevPot *P, const double *w0, size_t N, double dt, int64_
         a.dt = dt;
         a.first = k == 0;
         a.last = k == nchunk - 1;
-        if (lf_rows(LAY, N, n_steps, true))
+        if (rows)
             launch_rows(P, a, s);
         else
             hipLaunchKernelGGL((k_leapfrog_chunk<SCF, LAY>), dim3(g), dim3(LF_BLOCK), 0, s, P, a);
@@ -518,6 +516,7 @@ extern "C" int gamd_leapfrog_stream(const gamd_potential *pot, const double *w0,
         GAMD_HIP_CHECK(hipStreamSynchronize(s));
         return GAMD_OK;
     }
+    const bool rows = lf_rows(pot->dev.layout, N, n_steps, true);
     hipStream_t c = nullptr, cs = nullptr;
     hipEvent_t comp = nullptr, copied[2] = {nullptr, nullptr};
     hipGraph_t graph = nullptr;
@@ -531,8 +530,8 @@ extern "C" int gamd_leapfrog_stream(const gamd_potential *pot, const double *w0,
         hipEventCreateWithFlags(&copied[1], hipEventDisableTiming) != hipSuccess)
         goto done;
     if (!use_graph) {
-        rc = run(pot->ddev, w0, N, dt, n_steps, save_stride, chunk_rows, host_out, w_final, ring,
-                 state, s, c, comp, copied);
+        rc = run(pot->ddev, w0, N, dt, n_steps, save_stride, chunk_rows, rows, host_out, w_final,
+                 ring, state, s, c, comp, copied);
         // the events and the copy stream are released below: finish first
         if (rc == GAMD_OK && hipStreamSynchronize(s) != hipSuccess) rc = GAMD_ERR_HIP;
     } else {
@@ -542,8 +541,8 @@ extern "C" int gamd_leapfrog_stream(const gamd_potential *pot, const double *w0,
         // stream, after its earlier work
         if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) goto done;
         if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) goto done;
-        rc = run(pot->ddev, w0, N, dt, n_steps, save_stride, chunk_rows, host_out, w_final, ring,
-                 state, cs, c, comp, copied);
+        rc = run(pot->ddev, w0, N, dt, n_steps, save_stride, chunk_rows, rows, host_out, w_final,
+                 ring, state, cs, c, comp, copied);
         const hipError_t ce = hipStreamEndCapture(cs, &graph);
         if (rc != GAMD_OK || ce != hipSuccess || !graph) {
             rc = GAMD_ERR_HIP;

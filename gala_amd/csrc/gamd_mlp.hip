@@ -881,7 +881,9 @@ __global__ __launch_bounds__(256, 2) void k_train_tile(
 // points of one unit per lane).  Rows are padded by 32 bytes, which spreads
 // the 16 rows of a transposed read over all banks.
 constexpr int WG_P = 64;                            // points per stage
-constexpr int WG_SLICES = 42;                       // 3 layers x 2 halves x 42: one round of 256 CUs
+// 3 layers x 2 halves x 42: one round of 256 compute units.  Fixed: the order of the sums and the
+// size of the workspace are the same on every device.
+constexpr int WG_SLICES = 42;
 constexpr int WG_LA = H + 16, WG_LB = H / 2 + 16;   // LDS row lengths
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));

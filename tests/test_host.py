@@ -31,6 +31,26 @@ def test_library_exports_every_declared_symbol():
     assert _lib.load().gamd_version().startswith(b"gala_amd")
 
 
+@pytest.mark.parametrize("cus", [256, 128, 32])
+def test_dispatch_limits_follow_the_compute_units(cus, tmp_path):
+    """Rows of 16 lanes are taken while their waves (four rows each) have a SIMD
+    for themselves, final states to half of that, and rows are kept filled up to
+    one wave of single lanes to a SIMD: four SIMDs to a compute unit of any chip
+    or partition."""
+    simds = 4 * cus
+    src = tmp_path / "limits.cpp"
+    src.write_text(f"""
+#include "gamd_rules.hpp"
+static_assert(gamd::leapfrog_row_orbits({cus}, true) == {4 * simds}, "");
+static_assert(gamd::leapfrog_row_orbits({cus}, false) == {2 * simds}, "");
+static_assert(gamd::filled_row_orbits({cus}) == {64 * simds}, "");
+""")
+    csrc = os.path.join(ROOT, "gala_amd", "csrc")
+    r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", csrc, str(src)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+
 def test_invalid_arguments_are_rejected_without_gpu_work():
     """Argument checks happen before any HIP call."""
     from gala_amd import _lib
