@@ -5,15 +5,12 @@
 
 namespace gamd {
 
-// llvm.amdgcn.update.dpp on a double: one v_mov_b64_dpp (the builtin takes 32 bits)
-__device__ double dpp_f64(double old, double v, int ctrl, int row_mask, int bank_mask,
-                          bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.f64");
-
 template <int SRC>
 __device__ __forceinline__ double row_bcast(double v) {
     // DPP row_newbcast:SRC: every lane of a 16-lane row reads lane SRC of the
-    // row (every lane has a source in its row, so the zero is not used)
-    return dpp_f64(0.0, v, 0x150 + SRC, 0xF, 0xF, true);
+    // row (every lane has a source in its row, so the zero is not used); of a
+    // double one v_mov_b64_dpp
+    return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + SRC, 0xF, 0xF, true);
 }
 
 // The Milky-Way evaluator (mw_factors) on a 16-lane row whose lanes 0 to 7

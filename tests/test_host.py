@@ -51,6 +51,15 @@ static_assert(gamd::filled_row_orbits({cus}) == {64 * simds}, "");
     assert r.returncode == 0, r.stderr
 
 
+def test_kernels_reach_instructions_by_builtins_and_assembly_only():
+    """No device function borrows a compiler intrinsic's name by an asm label:
+    nothing promises that such a call is still the intrinsic."""
+    csrc = os.path.join(ROOT, "gala_amd", "csrc")
+    for f in sorted(os.listdir(csrc)):
+        text = open(os.path.join(csrc, f)).read()
+        assert not re.search(r'asm(__)?\s*\(\s*"llvm\.', text), f
+
+
 def test_invalid_arguments_are_rejected_without_gpu_work():
     """Argument checks happen before any HIP call."""
     from gala_amd import _lib
