@@ -170,6 +170,41 @@ def test_gradients_count_every_tile_once(M):
         close((sum(p[0] for p in parts), sum(p[1] for p in parts) / tiles), whole)
 
 
+@pytest.mark.parametrize("M", [2688, 2752, 5440])
+def test_gradients_of_uneven_batches(M):
+    """42, 43 and 85 tiles, where the batch in reverse order would not show a
+    loss that is the same from both ends.  Moved on by one tile (every tile's
+    points in another workgroup, stage and slice) the batch gives the same
+    gradient up to the order of the sums, M 2^-24; and two sub-batches of a third
+    and two thirds, weighted by their sizes, make up the whole up to the BF16
+    rounding of their signals, which 1 / M scales differently: 0.8 % at most in a
+    CPU simulation of these sizes, where one tile of 85 lost is 2.9 % or more.
+    The bar between them is 1 / 85, one tile's share."""
+    from gala_amd import _device as dev
+    t = dev.torch()
+    sur, pot, S, T = _surrogate(4)
+    rng = np.random.default_rng(M)
+    feat = dev.to_dev(rng.normal(size=(M, 4)), dtype=t.float32)
+    target = dev.to_dev(rng.normal(size=(M, 4)), dtype=t.float32)
+
+    def run(f, y):
+        loss, g = sur.gradients(f.contiguous(), y.contiguous())
+        return float(loss.item()), dev.to_host(g).astype(np.float64)
+
+    def close(a, b, bar):
+        assert abs(a[0] - b[0]) <= M * 2.0 ** -24 * b[0]
+        for (name, _), i, j in zip(OM.SHAPES, offsets[:-1], offsets[1:]):
+            rel = np.linalg.norm(a[1][i:j] - b[1][i:j]) / np.linalg.norm(b[1][i:j])
+            assert rel <= bar, (name, rel)
+
+    offsets = np.cumsum([0] + [int(np.prod(s)) for _, s in OM.SHAPES])
+    whole = run(feat, target)
+    close(run(feat.roll(64, 0), target.roll(64, 0)), whole, M * 2.0 ** -24)
+    k = M // 64 // 3 * 64
+    a, b = run(feat[:k], target[:k]), run(feat[k:], target[k:])
+    close((a[0] + b[0], (a[1] * k + b[1] * (M - k)) / M), whole, 1.0 / 85.0)
+
+
 def test_training_beats_monopole_and_falls_back():
     """A short training run: the loss falls, the trained network's force
     -grad Phi_net beats the monopole-only approximation (the method without
