@@ -152,7 +152,7 @@ __device__ __forceinline__ void net_physics(const gamd_mlp_norm &nm, double x, d
 // exactly those its reverse-pass products need.  All 256 threads call it.
 //
 // What bounds it: the matrix products and the SiLU arithmetic (1,152 MFMAs,
-// 18.4k cycles, and ~3,000 other vector instructions, ~15k cycles, per wave
+// 18.4k cycles, and ~2,700 other vector instructions, ~14k cycles, per wave
 // and 32-point tile), with the weights' L2 reads (1.5 MB per tile) close
 // behind.  1,048,576 points take 2.41 ms, 1,040 TFLOP/s of executed BF16
 // products (a large library BF16 product reaches 1,150 on the same card); 3.91
@@ -519,13 +519,13 @@ __global__ __launch_bounds__(256, 2) void k_mlp_forward(const float *__restrict_
 // slices of the points into partial matrices; k_grad_reduce adds slices and
 // tile rows in a fixed order, so gradients are the same in every run.
 //
-// 32,768 points: k_train_tile 61 us, k_wgrad 27, k_grad_reduce 9 and Adam 6;
-// 104 us per step end to end.  The same step took 450 us as twenty launches:
+// 32,768 points: k_train_tile 61 us, k_wgrad 26, k_grad_reduce 9 and Adam 5;
+// 112 to 118 us per step end to end.  The same step took 450 us as twenty launches:
 // a forward pass that wrote every pre-activation and activation (134 MB), a
 // product per layer that read them back, and reductions over the points by
 // atomic adds from every block (50 us per weight gradient, 31 us for dW5).
-// k_train_tile is bound by its vector work (~5,500 instructions and 768
-// exp2/rcp per wave, two waves per SIMD) beside 100 MB of stores; k_wgrad and
+// k_train_tile is bound by its vector work (~7,700 instructions per wave beside 768
+// matrix ones, two waves per SIMD: VALU 52 % busy) beside 100 MB of stores; k_wgrad and
 // k_grad_reduce by their 180 and 39 MB.  64-point tiles of four waves let two
 // workgroups share a compute unit, one's products behind the other's SiLU.
 
